@@ -27,7 +27,8 @@ MFMA_VGPR = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 SOURCES = [("k_quant.hip", "k_quant", []), ("k_ops.hip", "k_ops", []), ("runtime.cpp", "runtime", []),
            ("gemv_dispatch.cpp", "gemv_dispatch", []), ("k_qgemm.hip", "k_qgemm", MFMA_VGPR),
            ("k_attn_prefill.hip", "k_attn_prefill", MFMA_VGPR), ("gguf.cpp", "gguf", []), ("smq.cpp", "smq", []), ("host_common.cpp", "host_common", []), ("k_sample.hip", "k_sample", [])] + [
-           ("k_gemv.hip", f"k_gemv_f{f}", [f"-DSMX_GEMV_FMT={f}"]) for f in range(9)]
+           ("k_gemv.hip", f"k_gemv_f{f}", [f"-DSMX_GEMV_FMT={f}"]) for f in range(9)] + [
+           ("k_qgemm_tile.hip", f"k_qgemm_tile_f{f}", [f"-DSMX_TILE_FMT={f}", *MFMA_VGPR]) for f in (0, 1, 2, 3, 4, 7, 8)]
 
 FLAGS = [
     "-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "-fvisibility=hidden",

@@ -73,7 +73,7 @@ __device__ __forceinline__ float rows_sum(float v)
 __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
     const float *__restrict__ q, int q_stride, const float *__restrict__ kc, const float *__restrict__ vc,
     float *__restrict__ out, int out_stride, int n_head, int n_kv_head, int ctx_stride, int p_first, int M,
-    uint8_t *__restrict__ out_parts, int tok_off, PrefillBlocks pb)
+    uint8_t *__restrict__ out_parts, int tok_off, XpSums sums, PrefillBlocks pb)
 {
     extern __shared__ float s_out[];          // [kWaves][kRows][kPitch]
     __shared__ float s_max[kWaves][kRows], s_sum[kWaves][kRows], s_inv[kRows];
@@ -248,6 +248,13 @@ __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
             xp_store(out_parts, nsb, tok_off + t, k + 1, acc.y);
             xp_store(out_parts, nsb, tok_off + t, k + 2, acc.z);
             xp_store(out_parts, nsb, tok_off + t, k + 3, acc.w);
+            if (sums.kind) {   // the 8 threads of a 32-dimension sub-block are neighbouring lanes
+                float q = (acc.x + acc.y) + (acc.z + acc.w);
+                q += dpp_mov<0xB1>(q);
+                q += dpp_mov<0x4E>(q);                    // 16 dimensions
+                const float o = dpp_mov<0x141>(q);        // the other quad's
+                if ((tid & 7) == 0) xp_sums(out_parts, sums.kind, sums.M, nsb, tok_off + t, k >> 5, q, o);
+            }
         } else {
             *(float4 *)(out + (int64_t)t * out_stride + (int64_t)h * kHD + d4) = acc;
         }
@@ -265,7 +272,8 @@ bool attention_prefill_supported(int n_head, int n_kv_head, int hd)
 
 hipError_t launch_attention_prefill(const float *q, int q_stride, const float *kc, const float *vc, float *out,
                                     int out_stride, int n_head, int n_kv_head, int hd, int ctx_stride,
-                                    int p_first, int M, hipStream_t s, uint8_t *out_parts, int tok_off)
+                                    int p_first, int M, hipStream_t s, uint8_t *out_parts, int tok_off,
+                                    XpSums sums)
 {
     if (!attention_prefill_supported(n_head, n_kv_head, hd) || M <= 0 || p_first < 0 || ((n_head * hd) & 31) ||
         p_first + M > ctx_stride || (q_stride & 3) || (out_stride & 3) || tok_off < 0)
@@ -277,7 +285,7 @@ hipError_t launch_attention_prefill(const float *q, int q_stride, const float *k
     const int TT = kRows / (n_head / n_kv_head);
     const dim3 grid((unsigned)((M + TT - 1) / TT), (unsigned)n_kv_head);
     hipLaunchKernelGGL(k_attn_prefill, grid, dim3(kWaves * 64), lds, s, q, q_stride, kc, vc, out, out_stride,
-                       n_head, n_kv_head, ctx_stride, p_first, M, out_parts, tok_off, PrefillBlocks{});
+                       n_head, n_kv_head, ctx_stride, p_first, M, out_parts, tok_off, sums, PrefillBlocks{});
     return hipGetLastError();
 }
 
@@ -285,7 +293,7 @@ int attention_prefill_block_rows(int n_head, int n_kv_head) { return kRows / (n_
 
 hipError_t launch_attention_prefill_blocks(const float *q, int q_stride, float *out, int out_stride, int n_head,
                                            int n_kv_head, int hd, int ctx_stride, int n_blocks,
-                                           const PrefillBlocks &pb, hipStream_t s, uint8_t *out_parts)
+                                           const PrefillBlocks &pb, hipStream_t s, uint8_t *out_parts, XpSums sums)
 {
     if (!attention_prefill_supported(n_head, n_kv_head, hd) || n_blocks <= 0 || !pb.blk || !pb.kc_tok ||
         !pb.vc_tok || !pb.pos || ((n_head * hd) & 31) || (q_stride & 3) || (out_stride & 3))
@@ -296,7 +304,7 @@ hipError_t launch_attention_prefill_blocks(const float *q, int q_stride, float *
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)n_blocks, (unsigned)n_kv_head);
     hipLaunchKernelGGL(k_attn_prefill, grid, dim3(kWaves * 64), lds, s, q, q_stride, nullptr, nullptr, out,
-                       out_stride, n_head, n_kv_head, ctx_stride, 0, 0, out_parts, 0, pb);
+                       out_stride, n_head, n_kv_head, ctx_stride, 0, 0, out_parts, 0, sums, pb);
     return hipGetLastError();
 }
 

@@ -787,7 +787,8 @@ template <int HD>
 __global__ __launch_bounds__(AttnCfg<HD>::NT) void k_attention_tokens(
     const float *__restrict__ q, int64_t q_stride, float *const *__restrict__ kc_tok,
     float *const *__restrict__ vc_tok, int64_t layer_off, float *__restrict__ out, int64_t out_stride,
-    int n_head, int n_kv_head, int ctx_stride, const int32_t *__restrict__ tok_pos, uint8_t *__restrict__ out_parts)
+    int n_head, int n_kv_head, int ctx_stride, const int32_t *__restrict__ tok_pos, uint8_t *__restrict__ out_parts,
+    XpSums sums)
 {
     constexpr int NT = AttnCfg<HD>::NT;
     extern __shared__ float4 smem4[];
@@ -800,7 +801,7 @@ __global__ __launch_bounds__(AttnCfg<HD>::NT) void k_attention_tokens(
     attention_head<HD, NT, AttnCfg<HD>::U>(q + (int64_t)t * q_stride + (int64_t)h * HD, kc_tok[t] + off,
                                            vc_tok[t] + off, out + (int64_t)t * out_stride + (int64_t)h * HD,
                                            n_pos, ctx_stride, (float *)smem4, sm, out_parts, n_head * HD / 32, t,
-                                           h * HD);
+                                           h * HD, sums);
 }
 
 // Argmax of each row of logits [M][n] (lowest index on ties); with `tok_arr`, appends the
@@ -1079,9 +1080,9 @@ hipError_t launch_attention_tokens(const float *q, int64_t q_stride, float *cons
                                    float *const *vc_tok, int64_t layer_off, float *out,
                                    int64_t out_stride, int n_head, int n_kv_head, int hd,
                                    int ctx_stride, const int32_t *tok_pos, int M, hipStream_t s,
-                                   uint8_t *out_parts)
+                                   uint8_t *out_parts, XpSums sums)
 {
-    if (out_parts && (n_head * hd) % 32) return hipErrorInvalidValue;
+    if (out_parts && ((n_head * hd) % 32 || (sums.kind && hd < 32))) return hipErrorInvalidValue;
     const size_t lds = (size_t)ctx_stride * 4;
     const void *fn = nullptr;
     switch (hd) {
@@ -1096,7 +1097,7 @@ hipError_t launch_attention_tokens(const float *q, int64_t q_stride, float *cons
         if (e != hipSuccess) return e;
     }
     const dim3 grid((unsigned)n_head, (unsigned)M);
-#define SMX_ATT_T(HD) hipLaunchKernelGGL(k_attention_tokens<HD>, grid, dim3(AttnCfg<HD>::NT), lds, s, q, q_stride, kc_tok, vc_tok, layer_off, out, out_stride, n_head, n_kv_head, ctx_stride, tok_pos, out_parts)
+#define SMX_ATT_T(HD) hipLaunchKernelGGL(k_attention_tokens<HD>, grid, dim3(AttnCfg<HD>::NT), lds, s, q, q_stride, kc_tok, vc_tok, layer_off, out, out_stride, n_head, n_kv_head, ctx_stride, tok_pos, out_parts, sums)
     switch (hd) {
     case 16: SMX_ATT_T(16); break;
     case 32: SMX_ATT_T(32); break;

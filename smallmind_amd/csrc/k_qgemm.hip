@@ -1,6 +1,8 @@
 // k_qgemm.hip -- quantized GEMM Y[M][N] = X[M][K] . W[N][K]^T on the bf16 matrix cores, for
-// several activation rows at once (m >= 16: batched decode of many sessions, prefill chunks,
-// IWeightTensor.MatMul with m > 1; NeuralNet.cs:145-298, MatMulF32Q8.cs:23-80).
+// several activation rows at once (batched decode of many sessions, short prompts,
+// IWeightTensor.MatMul with m > 1; NeuralNet.cs:145-298, MatMulF32Q8.cs:23-80), the preparation of
+// its activation parts, and the dispatch between these kernels and the tile kernel for longer
+// prompts (k_qgemm_tile.hip, qgemm_tiled).
 //
 // Exactness.  The MFMA inputs are bf16, the reference computes in fp32.  Both sides are made
 // exact:
@@ -29,351 +31,13 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "smx_device.h"
-#include "smx_formats.h"
-#include "smx_internal.h"
+#include "smx_qgemm.h"
 
 namespace smx {
 
+hipError_t launch_qgemm_tile(const QgemmArgs &a, hipStream_t s);
+
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ bf16x8 as_bf16x8(uint4 v)
-{
-    bf16x8 r;
-    __builtin_memcpy(&r, &v, 16);
-    return r;
-}
-
-__device__ __forceinline__ f32x4 mfma(uint4 a, uint4 b, f32x4 c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
-}
-
-// bf16 of an fp32 holding an integer of at most 8 significant bits (exact: the low 16 bits are 0)
-__device__ __forceinline__ uint32_t pack_hi16(float lo, float hi)
-{
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-
-// (a & m) | (b & ~m) and the bf16 pair 128 + (e & m) per 16-bit half, one v_bitop3_b32 each
-// (truth-table index = 4 * bit of the first operand + 2 * second + third)
-__device__ __forceinline__ uint32_t bfi(uint32_t m, uint32_t a, uint32_t b)
-{
-    return __builtin_amdgcn_bitop3_b32(a, m, b, 0xE2);   // m ? a : b
-}
-__device__ __forceinline__ uint32_t code_pair(uint32_t e, uint32_t m)
-{
-    return __builtin_amdgcn_bitop3_b32(e, m, 0x43004300u, 0xEA);   // (e & m) | 0x43004300
-}
-
-// ---- per-format weight operand --------------------------------------------------------------
-// load(): the raw words of (row, sub-block s, k-group g) -- codes and scale fields -- issued
-// one sub-block ahead of use; codes(): 4 bf16 pairs (element p, element p + 4) of the group's
-// 8 codes; scale(): the per-(row, sub-block) scale terms.
-struct RawQ {
-    uint4 h;          // K-quant super-block header
-    uint32_t v, v2;   // code bytes of the group
-    uint32_t H, H2;   // high bits (Q5_K: qh'; Q6_K: D0, D1)
-    uint32_t d;       // fp16 scale (Q4_0, Q8_0, Q6_K) / Q6_K int8 scale pair in the high half
-};
-struct Scl {
-    float sc, sc2, m;   // Q6_K uses sc (first 16 elements) and sc2 (second 16)
-};
-
-template <int F> struct QW;
-
-// Q4_0: block = sub-block of 32; codes n ^ 8 (value = code - 8): offset 128 + 8.
-template <> struct QW<FMT_Q4_0> {
-    static constexpr float kOff = 136.0f;
-    static constexpr bool kHalves = false;
-    __device__ __forceinline__ static RawQ load(const WView &w, uint32_t row, int s, int g)
-    {
-        RawQ r{};
-        const uint32_t blk = row * (uint32_t)w.nb + (uint32_t)s;
-        r.v = *(const uint32_t *)(w.q + blk * 16u + 4u * g);
-        r.d = w.d[blk];
-        return r;
-    }
-    __device__ __forceinline__ static uint4 codes(const RawQ &r, int)
-    {
-        const uint32_t v = r.v ^ 0x88888888u;
-        return make_uint4((v & 0x000F000Fu) | 0x43004300u, ((v >> 4) & 0x000F000Fu) | 0x43004300u,
-                          ((v >> 8) & 0x000F000Fu) | 0x43004300u, ((v >> 12) & 0x000F000Fu) | 0x43004300u);
-    }
-    __device__ __forceinline__ static Scl scale(const RawQ &r, int) { return {h2f(r.d), 0.0f, 0.0f}; }
-};
-
-// Q8_0: int8 codes; bf16(b ^ 0x80) = value + 128 (exact integers up to 255).
-template <> struct QW<FMT_Q8_0> {
-    static constexpr float kOff = 128.0f;
-    static constexpr bool kHalves = false;
-    __device__ __forceinline__ static RawQ load(const WView &w, uint32_t row, int s, int g)
-    {
-        RawQ r{};
-        const uint32_t blk = row * (uint32_t)w.nb + (uint32_t)s;
-        const uint2 v = *(const uint2 *)(w.q + blk * 32u + 8u * g);
-        r.v = v.x;
-        r.v2 = v.y;
-        r.d = w.d[blk];
-        return r;
-    }
-    __device__ __forceinline__ static uint4 codes(const RawQ &r, int)
-    {
-        const uint32_t a = r.v ^ 0x80808080u, b = r.v2 ^ 0x80808080u;
-        // pair p = (element p, element p + 4) = (byte p of a, byte p of b)
-        float a0, a1, a2, a3, b0, b1, b2, b3;
-        asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(a0) : "v"(a));
-        asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(a1) : "v"(a));
-        asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(a2) : "v"(a));
-        asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(a3) : "v"(a));
-        asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(b0) : "v"(b));
-        asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(b1) : "v"(b));
-        asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(b2) : "v"(b));
-        asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(b3) : "v"(b));
-        return make_uint4(pack_hi16(a0, b0), pack_hi16(a1, b1), pack_hi16(a2, b2), pack_hi16(a3, b3));
-    }
-    __device__ __forceinline__ static Scl scale(const RawQ &r, int) { return {h2f(r.d), 0.0f, 0.0f}; }
-};
-
-// SMQ blocks (Q8Tensor / Q4Tensor): the Q8_0 / Q4_0 codes with an fp32 scale per 32 elements.
-template <> struct QW<FMT_SQ8> {
-    static constexpr float kOff = 128.0f;
-    static constexpr bool kHalves = false;
-    __device__ __forceinline__ static RawQ load(const WView &w, uint32_t row, int s, int g)
-    {
-        RawQ r{};
-        const uint32_t blk = row * (uint32_t)w.nb + (uint32_t)s;
-        const uint2 v = *(const uint2 *)(w.q + blk * 32u + 8u * g);
-        r.v = v.x;
-        r.v2 = v.y;
-        r.d = ((const uint32_t *)w.d)[blk];
-        return r;
-    }
-    __device__ __forceinline__ static uint4 codes(const RawQ &r, int g) { return QW<FMT_Q8_0>::codes(r, g); }
-    __device__ __forceinline__ static Scl scale(const RawQ &r, int) { return {__uint_as_float(r.d), 0.0f, 0.0f}; }
-};
-
-template <> struct QW<FMT_SQ4> {
-    static constexpr float kOff = 136.0f;
-    static constexpr bool kHalves = false;
-    __device__ __forceinline__ static RawQ load(const WView &w, uint32_t row, int s, int g)
-    {
-        RawQ r{};
-        const uint32_t blk = row * (uint32_t)w.nb + (uint32_t)s;
-        r.v = *(const uint32_t *)(w.q + blk * 16u + 4u * g);
-        r.d = ((const uint32_t *)w.d)[blk];
-        return r;
-    }
-    __device__ __forceinline__ static uint4 codes(const RawQ &r, int g) { return QW<FMT_Q4_0>::codes(r, g); }
-    __device__ __forceinline__ static Scl scale(const RawQ &r, int) { return {__uint_as_float(r.d), 0.0f, 0.0f}; }
-};
-
-// Q4_K: sub-block s = qs bytes 16 + 16*(s % 8) of super-block s / 8.
-template <> struct QW<FMT_Q4_K> {
-    static constexpr float kOff = 128.0f;
-    static constexpr bool kHalves = false;
-    __device__ __forceinline__ static RawQ load(const WView &w, uint32_t row, int s, int g)
-    {
-        RawQ r{};
-        const uint32_t base = (row * (uint32_t)w.nb + ((uint32_t)s >> 3)) * 144u;
-        r.h = *(const uint4 *)(w.q + base);
-        r.v = *(const uint32_t *)(w.q + base + 16u + 16u * ((uint32_t)s & 7u) + 4u * g);
-        return r;
-    }
-    __device__ __forceinline__ static uint4 codes(const RawQ &r, int)
-    {
-        const uint32_t v = r.v;
-        return make_uint4((v & 0x000F000Fu) | 0x43004300u, ((v >> 4) & 0x000F000Fu) | 0x43004300u,
-                          ((v >> 8) & 0x000F000Fu) | 0x43004300u, ((v >> 12) & 0x000F000Fu) | 0x43004300u);
-    }
-    __device__ __forceinline__ static Scl scale(const RawQ &r, int s)
-    {
-        const int j = s & 7;
-        return {h2f(r.h.x & 0xFFFFu) * (float)kq_scale6(r.h.y, r.h.z, r.h.w, j, 0), 0.0f,
-                h2f(r.h.x >> 16) * (float)kq_scale6(r.h.y, r.h.z, r.h.w, j, 1)};
-    }
-};
-
-// Q5_K: codes = ql nibble | high bit (bit-permuted qh'), value = q - 16: offset 128 + 16.
-template <> struct QW<FMT_Q5_K> {
-    static constexpr float kOff = 144.0f;
-    static constexpr bool kHalves = false;
-    __device__ __forceinline__ static RawQ load(const WView &w, uint32_t row, int s, int g)
-    {
-        RawQ r{};
-        const uint32_t base = (row * (uint32_t)w.nb + ((uint32_t)s >> 3)) * 176u;
-        const uint32_t j = (uint32_t)s & 7u;
-        r.h = *(const uint4 *)(w.q + base);
-        r.v = *(const uint32_t *)(w.q + base + 48u + 16u * j + 4u * g);
-        r.H = *(const uint32_t *)(w.q + base + 16u + 4u * j);
-        return r;
-    }
-    __device__ __forceinline__ static uint4 codes(const RawQ &r, int g)
-    {
-        // The high bit of element 8g + 2k + p sits at bit 8k + 2g + p of H, so hg = H >> 2g
-        // holds it at bit 8k + p.  e0 / e1 = the 5-bit codes of the even / odd elements
-        // 2k / 2k + 1 in bits 0-4 of byte k (bits 5-7 are don't-care); pair q = (element q,
-        // element q + 4) is then bytes 0 and 2 of e_{q%2} >> 8(q/2).
-        const uint32_t v = r.v, hg = r.H >> (2 * g);
-        const uint32_t e0 = bfi(0x0F0F0F0Fu, v, hg << 4), e1 = bfi(0x0F0F0F0Fu, v >> 4, hg << 3);
-        return make_uint4(code_pair(e0, 0x001F001Fu), code_pair(e1, 0x001F001Fu), code_pair(e0 >> 8, 0x001F001Fu),
-                          code_pair(e1 >> 8, 0x001F001Fu));
-    }
-    __device__ __forceinline__ static Scl scale(const RawQ &r, int s)
-    {
-        const int j = s & 7;
-        return {h2f(r.h.x & 0xFFFFu) * (float)kq_scale6(r.h.y, r.h.z, r.h.w, j, 0), 0.0f,
-                h2f(r.h.x >> 16) * (float)kq_scale6(r.h.y, r.h.z, r.h.w, j, 1)};
-    }
-};
-
-// Q6_K: 6-bit codes, value = q - 32: offset 128 + 32; two 16-element scales per sub-block.
-template <> struct QW<FMT_Q6_K> {
-    static constexpr float kOff = 160.0f;
-    static constexpr bool kHalves = true;
-    __device__ __forceinline__ static RawQ load(const WView &w, uint32_t row, int s, int g)
-    {
-        RawQ r{};
-        const uint32_t sb = row * (uint32_t)w.nb + ((uint32_t)s >> 3);
-        const uint32_t base = sb * 208u, cc = (uint32_t)s & 7u;
-        r.v = *(const uint32_t *)(w.q + base + 16u * cc + 4u * g);
-        const uint2 D = *(const uint2 *)(w.q + base + 128u + 8u * cc);
-        r.H = D.x;
-        r.H2 = D.y;
-        r.d = (uint32_t)w.d[sb] | ((uint32_t)*(const uint16_t *)(w.q + base + 192u + 2u * cc) << 16);
-        return r;
-    }
-    __device__ __forceinline__ static uint4 codes(const RawQ &r, int g)
-    {
-        // The two high bits of element 8g + 2k + p sit at bits 8k + 2g of D_p, so
-        // dp = D_p >> 2g holds them at bits 8k, 8k + 1: e_p = the 6-bit codes of the elements
-        // 2k + p in bits 0-5 of byte k, and pair q = bytes 0 and 2 of e_{q%2} >> 8(q/2).
-        const uint32_t v = r.v;
-        const uint32_t e0 = bfi(0x0F0F0F0Fu, v, (r.H >> (2 * g)) << 4);
-        const uint32_t e1 = bfi(0x0F0F0F0Fu, v >> 4, (r.H2 >> (2 * g)) << 4);
-        return make_uint4(code_pair(e0, 0x003F003Fu), code_pair(e1, 0x003F003Fu), code_pair(e0 >> 8, 0x003F003Fu),
-                          code_pair(e1 >> 8, 0x003F003Fu));
-    }
-    __device__ __forceinline__ static Scl scale(const RawQ &r, int)
-    {
-        const float d = h2f(r.d & 0xFFFFu);
-        return {d * (float)(int8_t)((r.d >> 16) & 0xFFu), d * (float)(int8_t)(r.d >> 24), 0.0f};
-    }
-};
-
-constexpr uint4 kZero4 = {0u, 0u, 0u, 0u};
-
-// acc + sc * (C - off * sum x) - m * sum x as two fused steps: acc + sc*C - (sc*off + m) * sum x
-// (cs = sc * off + m precomputed per row and sub-block).
-// Activation part p of (token tile tt, sub-block s) for this lane: a wave-uniform base plus the
-// lane's 32-bit byte offset, so each load is one scalar-base instruction with no per-lane
-// 64-bit address arithmetic.
-__device__ __forceinline__ uint4 ld_part(const uint8_t *xp, int tt, int nsb, int s, int p, uint32_t lane16)
-{
-    const uint8_t *base = xp + (((size_t)tt * nsb + s) * 3 + p) * 1024;
-    return *(const uint4 *)(base + lane16);
-}
-
-__device__ __forceinline__ float accumulate1(float acc, float sc, float cs, float c, float sx)
-{
-    return __builtin_fmaf(sc, c, __builtin_fmaf(-cs, sx, acc));
-}
-// Two 16-element halves with their own scales (Q6_K): acc + sc*(Ca - off*sa) + sc2*(Cb - off*sb).
-__device__ __forceinline__ float accumulate2(float acc, float sc, float sc2, float ca, float cb, float sa, float sb,
-                                             float off)
-{
-    acc = __builtin_fmaf(-(sc * off), sa, acc);
-    acc = __builtin_fmaf(-(sc2 * off), sb, acc);
-    acc = __builtin_fmaf(sc, ca, acc);
-    return __builtin_fmaf(sc2, cb, acc);
-}
-constexpr uint32_t kOnes = 0x3F803F80u;   // bf16 1.0 pair
-
-// Inputs of the EPI_QKV epilogue for one (token, row) value, loaded by the caller ahead of the
-// epilogue: the token's position, the RoPE factors of the row's pair (when it is rotated) and
-// the token's K or V cache base (for K / V rows).
-struct QkvPre {
-    uint32_t pos;   // never negative: widening it is a zero extension, which waits for no load
-    float c, sn;
-    float *cache;
-};
-
-// Epilogue of one output value per (token, weight row); all lanes of the wave must call it
-// (adjacent weight rows are exchanged with DPP for the paired SwiGLU / RoPE epilogues).
-// Returns the new residual value for EPI_RESID with a.np set (0 for rows / tokens outside the
-// output), else 0.  With pre, EPI_RESID takes the residual and the next norm's gamma from
-// pres / pg, and EPI_QKV its position, RoPE factors and cache base from qp (all loaded by the
-// caller before the epilogue) instead of loading them here, so the epilogue's stores do not
-// wait for loads: vector-memory waits count stores as well, so a load between two stores
-// would also wait for the first store.
-__device__ __forceinline__ float qgemm_epilogue(const QgemmArgs &a, float v, uint32_t row, int tok, bool live,
-                                                bool pre = false, float pres = 0.0f, float pg = 0.0f,
-                                                QkvPre qp = QkvPre{0, 0.0f, 0.0f, nullptr})
-{
-    const uint32_t N = (uint32_t)a.w.rows;
-    if (a.bias && row < N) v = v + a.bias[row];
-    // value of the neighbouring weight row (lane li ^ 1 holds row ^ 1)
-    const float nb = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
-    if (!live || row >= N || tok >= a.M) return 0.0f;
-    float *yr = a.y + (int64_t)tok * a.y_stride;
-    switch (a.epi) {
-    case EPI_STORE: yr[row] = v; break;
-    case EPI_RESID: {
-        const float xn = (pre ? pres : yr[row]) + v;
-        yr[row] = xn;
-        if (a.np) {   // the next GEMM's parts of gamma (.) x (RMSNormOps.cs:137-139 up to the factor r)
-            xp_store(a.np, (int)(N >> 5), tok, (int)row, (pre ? pg : a.ngamma[row]) * xn);
-            return xn;
-        }
-        break;
-    }
-    case EPI_GELU:
-        if (a.yp) xp_store(a.yp, (int)(N >> 5), tok, (int)row, gelu_pade(v));
-        else yr[row] = gelu_pade(v);
-        break;
-    case EPI_SILU:
-        // rows interleave gate / up: out[i] = silu(gate_i) * up_i
-        if (!(row & 1)) {
-            const float y = silu_mul(v, nb);
-            if (a.yp) xp_store(a.yp, (int)(N >> 6), tok, (int)(row >> 1), y);
-            else yr[row >> 1] = y;
-        }
-        break;
-    case EPI_QKV: {
-        if (row & 1) break;
-        const int d = a.d_model, kv = a.kv_dim, hd = a.head_dim, r = (int)row;
-        const uint32_t pos = pre ? qp.pos : (uint32_t)a.tok_pos[tok];
-        float v0 = v, v1 = nb;
-        if (a.use_rope && r < d + kv) {
-            const int pair = ((r < d ? r : r - d) % hd) / 2, half = hd / 2;
-            const float c = pre ? qp.c : a.rope_cos[(int64_t)pos * half + pair];
-            const float sn = pre ? qp.sn : a.rope_sin[(int64_t)pos * half + pair];
-            const float t0 = v0 * c, t1 = v1 * sn, t2 = v0 * sn, t3 = v1 * c;   // RotaryEmbedding.cs:115-116
-            v0 = t0 - t1;
-            v1 = t2 + t3;
-        }
-        if (r < d) {
-            yr[r] = v0;
-            yr[r + 1] = v1;
-        } else if (r < d + kv) {
-            float *dst = (pre ? qp.cache : a.kc_tok[tok]) + a.layer_off + (int64_t)(r - d) * a.ctx_stride + pos;
-            dst[0] = v0;
-            dst[a.ctx_stride] = v1;
-        } else {
-            const int vr = r - d - kv;
-            float *dst = (pre ? qp.cache : a.vc_tok[tok]) + a.layer_off + ((int64_t)(vr / hd) * a.ctx_stride + pos) * hd + (vr % hd);
-            dst[0] = v0;
-            dst[1] = v1;
-        }
-        break;
-    }
-    default: break;
-    }
-    return 0.0f;
-}
 
 template <int F, int RT, int TT, int NW, int SB>
 __global__ __launch_bounds__(64 * NW) void k_qgemm(QgemmArgs a)
@@ -697,19 +361,6 @@ __device__ __forceinline__ RawQ stage_raw(const uint8_t *row, const uint32_t *dr
     return r;
 }
 
-// Tile order of a launch with several token-tile groups.  The 2-D grid (row tile x, token group
-// y) runs the row tiles fastest, and workgroups land on the 8 XCDs round robin, so each XCD works
-// on 1/8 of W for ~1.5 token groups at a time: W's slice plus those groups' activation parts
-// exceed the XCD's 4 MB L2, and W is fetched again for every token group.  With G > 0 the grid
-// is 1-D and workgroup i runs tile t = (i % 8) * chunk + i / 8 of a panel-major order (panels of
-// G token groups whose parts stay in the L2, row tiles in a panel with the G groups fastest), so
-// each XCD works through one contiguous chunk of that order: the parts of its panel stay
-// resident and each W tile is read once per panel by G workgroups in a row.
-struct TileSched {
-    uint32_t R, T;       // row tiles, token-tile groups
-    uint32_t G, chunk;   // groups per panel (0: the 2-D grid), tiles per XCD
-};
-
 // TS > 1 (one token tile only): the tile's 16 tokens are split over TS workgroups of 16 / TS
 // tokens each (grid y).  Each workgroup still multiplies whole 16 x 16 MFMA tiles, but it loads
 // the activation parts of its own tokens only (the other token lanes repeat them) and stores
@@ -717,7 +368,7 @@ struct TileSched {
 // most of what a one-token-tile workgroup moves into its CU, and the split also spreads a
 // matrix of few row tiles over more CUs.  No partial sums cross workgroups.
 template <int F, int RT, int TT, int NW, int TS = 1>
-__global__ __launch_bounds__(64 * NW) void k_qgemm_st(QgemmArgs a, TileSched ts)
+__global__ __launch_bounds__(64 * NW) void k_qgemm_st(QgemmArgs a)
 {
     static_assert(TS == 1 || (TT == 1 && (TS == 2 || TS == 4)), "token split of one token tile into 8 or 4");
     using Q = QW<F>;
@@ -738,19 +389,7 @@ __global__ __launch_bounds__(64 * NW) void k_qgemm_st(QgemmArgs a, TileSched ts)
     const uint32_t lane16 = (uint32_t)lane * 16u;
     const uint32_t N = (uint32_t)w.rows;
     const int nsb = (int)(w.cols >> 5), nsup = nsb >> 3;
-    uint32_t bx = blockIdx.x, by = blockIdx.y;
-    // one token tile (the lockstep step): never scheduled, and the latency-bound launch reads
-    // no schedule argument (reading and testing it cost 2 % of the configs[4] step)
-    if constexpr (TT > 1) {
-        if (ts.G) {   // wave-uniform: the whole workgroup takes the same branch
-            const uint32_t i = blockIdx.x, t = (i & 7u) * ts.chunk + (i >> 3);
-            if (t >= ts.R * ts.T) return;
-            const uint32_t pt = ts.R * ts.G, panel = t / pt, rem = t - panel * pt;
-            const uint32_t gp = min(ts.G, ts.T - panel * ts.G);
-            bx = rem / gp;
-            by = panel * ts.G + (rem - bx * gp);
-        }
-    }
+    const uint32_t bx = blockIdx.x, by = blockIdx.y;
     const uint32_t row_base = bx * R16;
     // token split: this workgroup's tokens are tlo .. tlo + TW - 1 of the single token tile
     constexpr int TW = 16 / TS;
@@ -1041,24 +680,8 @@ template <int F, int NR> struct RsSlot {
     uint4 w[NR * Stage<F>::kBytes];    // NR * 16 rows x kBytes, row-major, in 16-byte pieces
 };
 
+
 template <int N> using ic = std::integral_constant<int, N>;
-
-// 16 bytes per lane from global address g into LDS at l + 16 * lane (l wave-uniform; M0 holds
-// it, with the one wait state between the M0 write and the load)
-__device__ __forceinline__ void lds_dma16(const void *g, void *l)
-{
-    const uint32_t la = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)l;
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(la) : "memory");
-}
-
-// s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 6:4 left
-// alone, lgkmcnt 11:8): the wave's vector-memory loads older than its last n have landed and
-// its own LDS reads have completed
-template <int N> __device__ __forceinline__ void wait_vm_lds()
-{
-    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
-}
 
 template <int F, int NR, int NKH, int NS>
 __global__ __launch_bounds__(64 * NR * NKH) void k_qgemm_rs(QgemmArgs a)
@@ -1468,6 +1091,98 @@ __global__ __launch_bounds__(256) void k_qprep_long(const float *__restrict__ x,
     }
 }
 
+// More than 16 tokens: a workgroup takes 4 tokens (a quarter of a token tile), thread (item lane
+// tid / 4, token tid % 4).  Four neighbouring lanes store the same item of four tokens, 64
+// contiguous bytes of a part (one token per workgroup stored 16-byte pieces 256 bytes apart, which
+// ran at a third of the copy rate).  The rows of a norm are read again from the L1 for the
+// second pass instead of being held in registers.  SUMS: the kind of sub-block sums written (xp_sums).
+template <int PRO, int SUMS>
+__global__ __launch_bounds__(256) void k_qprep_tokens(const float *__restrict__ x, int64_t x_stride, int M, int K,
+                                                      const float *__restrict__ gamma,
+                                                      const float *__restrict__ beta, float eps,
+                                                      uint8_t *__restrict__ xp)
+{
+    __shared__ float red[4][4];
+    const int nsb = K >> 5, items = K >> 3, ntt = (M + 15) >> 4;
+    const int tid = threadIdx.x, tq = tid & 3, i0 = tid >> 2;
+    const int m = blockIdx.x * 4 + tq, tt = m >> 4, t = m & 15;
+    const bool live = m < M;
+    const float4 *xr = (const float4 *)(x + (int64_t)min(m, M - 1) * x_stride);
+    const float4 *g4 = (const float4 *)gamma, *b4 = (const float4 *)beta;
+    // sum over the row of this thread's token: lanes of equal tid % 4, then the four waves
+    auto row_sum = [&](float v) {
+#pragma unroll
+        for (int o = 4; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
+        __syncthreads();
+        if ((tid & 63) < 4) red[tid >> 6][tq] = v;
+        __syncthreads();
+        return (red[0][tq] + red[1][tq]) + (red[2][tq] + red[3][tq]);
+    };
+    float sc = 1.0f, mean = 0.0f;
+    if constexpr (PRO == PRO_LN) {
+        float s = 0.0f;
+#pragma unroll 4
+        for (int i = i0; i < items; i += 64) {
+            float v[8];
+            unpack8(xr[2 * i], xr[2 * i + 1], v);
+#pragma unroll
+            for (int k = 0; k < 8; k++) s += v[k];
+        }
+        mean = row_sum(s) / (float)K;
+    }
+    if constexpr (PRO != PRO_NONE) {
+        float s = 0.0f;
+#pragma unroll 4
+        for (int i = i0; i < items; i += 64) {
+            float v[8];
+            unpack8(xr[2 * i], xr[2 * i + 1], v);
+#pragma unroll
+            for (int k = 0; k < 8; k++) { const float dd = PRO == PRO_LN ? v[k] - mean : v[k]; const float q = dd * dd; s += q; }
+        }
+        sc = 1.0f / sqrtf(row_sum(s) / (float)K + eps);
+    }
+    uint8_t *xt = xp + (size_t)tt * nsb * 3072u + t * 16;
+#pragma unroll 2
+    for (int i = i0; i < items; i += 64) {
+        float v[8];
+        unpack8(xr[2 * i], xr[2 * i + 1], v);
+        if constexpr (PRO != PRO_NONE) {
+            float gg[8];
+            unpack8(g4[2 * i], g4[2 * i + 1], gg);
+            if constexpr (PRO == PRO_RMS) {
+#pragma unroll
+                for (int k = 0; k < 8; k++) v[k] = gg[k] * (v[k] * sc);
+            } else {
+                float be[8];
+                unpack8(b4[2 * i], b4[2 * i + 1], be);
+#pragma unroll
+                for (int k = 0; k < 8; k++) v[k] = __builtin_fmaf(gg[k], (v[k] - mean) * sc, be[k]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = live ? v[k] : 0.0f;   // padding rows of the last tile
+        const int s = i >> 2, g = i & 3;
+        if constexpr (SUMS != 0) {   // the items of a sub-block are four lanes 4 apart (all active together)
+            float q = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+            q += __shfl_xor(q, 4, 64);
+            const float o = __shfl_xor(q, 8, 64);
+            if (g == 0) xp_sums(xp, SUMS, 16 * ntt, nsb, m, s, q, o);
+        }
+        uint8_t *p = xt + (size_t)s * 3072u + g * 256;
+#pragma unroll
+        for (int pt = 0; pt < 3; pt++) {
+            uint32_t w[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {   // pair q = (element q, element q + 4)
+                w[q] = bf16_pair(v[q], v[q + 4]);
+                v[q] -= __uint_as_float(w[q] << 16);
+                v[q + 4] -= __uint_as_float(w[q] & 0xFFFF0000u);
+            }
+            *(uint4 *)(p + 1024 * pt) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+}
+
 template <int F, int RT, int TT, int NW, int SB>
 hipError_t launch_frt(const QgemmArgs &a, hipStream_t s)
 {
@@ -1484,19 +1199,7 @@ hipError_t launch_st(const QgemmArgs &a, hipStream_t s)
     const uint32_t T = TS > 1 ? (uint32_t)((a.M + 16 / TS - 1) / (16 / TS))
                               : (uint32_t)(((a.M + 15) / 16 + TT - 1) / TT);
     if (TS > 1 && a.M > 16) return hipErrorInvalidValue;
-    TileSched ts{R, T, 0, 0};
-    dim3 grid(R, T);
-    // From 1024 tokens: panels of G token groups whose activation parts (TT tiles x K/32
-    // sub-blocks x 3 KB each) fill ~1.5 MB of an XCD's 4 MB L2.  Measured (configs[3] Q8_0 at
-    // 2048 tokens): L2 fills 2-2.3x lower (gate/up 16x -> 8.6x the algorithmic bytes), kernel
-    // times 0-2 % lower; at 511 tokens the 2-D order is 2-5 % faster, so shorter chunks keep it.
-    if (TT > 1 && T > 1 && a.M >= 1024) {
-        const uint64_t group_bytes = (uint64_t)TT * (uint64_t)(a.w.cols / 32) * 3072u;
-        ts.G = (uint32_t)std::min<uint64_t>(T, std::max<uint64_t>(1, (3u << 19) / group_bytes));
-        ts.chunk = (R * T + 7) / 8;
-        grid = dim3(8 * ts.chunk, 1);
-    }
-    hipLaunchKernelGGL((k_qgemm_st<F, RT, TT, NW, TS>), grid, dim3(64 * NW), 0, s, a, ts);
+    hipLaunchKernelGGL((k_qgemm_st<F, RT, TT, NW, TS>), dim3(R, T), dim3(64 * NW), 0, s, a);
     return hipGetLastError();
 }
 
@@ -1512,16 +1215,14 @@ template <int F>
 hipError_t launch_f(const QgemmArgs &a, hipStream_t s)
 {
     // Rows of whole 256-element super-blocks: LDS-staged weight tiles.  Up to 16 tokens: one
-    // token tile per workgroup (16 waves splitting K from 8192 up).  More: per wave RT x 16
-    // rows by TT x 16 tokens, NW waves splitting K; chosen by measurement (matrix-core GEMM
-    // with its k_qprep, weights resident) at 256-token chunks and at the 512 / 2048-token
-    // chunks of the configs[2] / configs[3] prompts:
+    // token tile per workgroup (16 waves splitting K from 8192 up).  More tokens come here only
+    // while they make few tiles (qgemm_tiled): per wave RT x 16 rows by TT x 16 tokens, NW waves
+    // splitting K; chosen by measurement at 256- and 512-token chunks:
     //  - K-quants (Q4_K / Q5_K): tall matrices 64 rows x 32 tokens, 4 waves; few rows or long
     //    K (O, down) the same above 320 tokens (Q4_K O 47.8 -> 39.7 us, down 92.0 -> 82.0 at
     //    512), 32 x 64 with 8 waves up to 320; other shapes (QKV) 32 x 32, 4 waves (Q4_K QKV 52.5
     //    -> 45.9 us at 512, Q5_K 52.1 -> 50.4 at 256);
-    //  - Q8_0 / Q4_0 / SMQ: 32 x 64, 4 waves; few rows or long K with 8 waves below 1024
-    //    tokens (Q8_0 O 165 -> 131 us, down 346 -> 317 at 2048 tokens with 4);
+    //  - Q8_0 / Q4_0 / SMQ: 32 x 64, 4 waves; few rows or long K with 8 waves;
     //  - Q6_K: 32 x 64 with 8 waves on few rows or long K, else 16 x 64.
     if (a.w.cols % 256 == 0) {
         const bool tall = a.w.rows >= 8192;
@@ -1535,7 +1236,7 @@ hipError_t launch_f(const QgemmArgs &a, hipStream_t s)
             if constexpr (F == FMT_Q6_K) return narrow ? launch_st<F, 2, 4, 8>(a, s) : launch_st<F, 1, 4, 8>(a, s);
             // (SMQ Q8's two staged scale words per sub-block do not fit 8 waves' registers)
             if constexpr (F != FMT_SQ8)
-                if (narrow && a.M < 1024) return launch_st<F, 2, 4, 8>(a, s);
+                if (narrow) return launch_st<F, 2, 4, 8>(a, s);
             return launch_st<F, 2, 4, 4>(a, s);
         }
         // tall K-quant matrices up to one workgroup of 64 rows per CU: the row-split kernel
@@ -1586,7 +1287,53 @@ hipError_t launch_d(const QgemmArgs &a, hipStream_t s)
 
 }  // namespace
 
-size_t qgemm_xp_bytes(int M, int K) { return (size_t)(((int64_t)M + 15) / 16) * (size_t)(K / 32) * 3 * 1024; }
+size_t qgemm_parts_bytes(int M, int K) { return (size_t)(((int64_t)M + 15) / 16) * (size_t)(K / 32) * 3 * 1024; }
+
+// the parts, then up to two sums of three bf16 parts per token and sub-block (xp_sums): 1/16
+size_t qgemm_xp_bytes(int M, int K) { return qgemm_parts_bytes(M, K) / 16 * 17; }
+
+int64_t qgemm_tiles(const WView &w, int M) { return ((w.rows + 63) / 64) * (((int64_t)M + 63) / 64); }
+
+// With few 64 x 64 tiles the K-split kernel (16 x 16 tiles, up to 8 waves on one tile's K) fills the
+// chip better.  Measured per call, K-split / tile: 2048 x 2048 Q8_0 at 256 tokens (128 tiles) 31 / 34
+// us, at 384 tokens 44 / 36; Q6_K 34 / 39 and 53 / 42; Q4_K at 511 tokens (256 tiles) 38 / 39, 16384 x
+// 2048 at 128 tokens (512) 56 / 51, 2560 x 2048 at 511 (320) 44 / 47, at 700 (440) 54 / 52.  From 640
+// tokens (K-quants with mins, which the K-split kernel runs on larger tiles: 1024) the tile kernel is
+// level or ahead at every row count (768 x 768 at 700 tokens Q8_0 35 / 25, Q4_K at 1024 25 / 26).
+bool qgemm_tiled(const WView &w, int M)
+{
+    if (M <= 16 || w.cols % 256 != 0 || fmt_dense(w.fmt)) return false;
+    const bool mins = w.fmt == FMT_Q4_K || w.fmt == FMT_Q5_K;
+    return M >= (mins ? 1024 : 640) || qgemm_tiles(w, M) >= (mins ? 440 : 160);
+}
+
+int qgemm_sums_kind(const WView &w, int M)
+{
+    if (!qgemm_tiled(w, M) || w.fmt == FMT_Q8_0 || w.fmt == FMT_SQ8) return 0;   // signed codes: no offset, no min
+    return w.fmt == FMT_Q6_K ? 2 : 1;
+}
+
+hipError_t launch_qgemm_tile_f0(const QgemmArgs &a, hipStream_t s);
+hipError_t launch_qgemm_tile_f1(const QgemmArgs &a, hipStream_t s);
+hipError_t launch_qgemm_tile_f2(const QgemmArgs &a, hipStream_t s);
+hipError_t launch_qgemm_tile_f3(const QgemmArgs &a, hipStream_t s);
+hipError_t launch_qgemm_tile_f4(const QgemmArgs &a, hipStream_t s);
+hipError_t launch_qgemm_tile_f7(const QgemmArgs &a, hipStream_t s);
+hipError_t launch_qgemm_tile_f8(const QgemmArgs &a, hipStream_t s);
+
+hipError_t launch_qgemm_tile(const QgemmArgs &a, hipStream_t s)
+{
+    switch (a.w.fmt) {
+    case FMT_Q4_0: return launch_qgemm_tile_f0(a, s);
+    case FMT_Q8_0: return launch_qgemm_tile_f1(a, s);
+    case FMT_Q4_K: return launch_qgemm_tile_f2(a, s);
+    case FMT_Q5_K: return launch_qgemm_tile_f3(a, s);
+    case FMT_Q6_K: return launch_qgemm_tile_f4(a, s);
+    case FMT_SQ8: return launch_qgemm_tile_f7(a, s);
+    case FMT_SQ4: return launch_qgemm_tile_f8(a, s);
+    default: return hipErrorInvalidValue;
+    }
+}
 
 hipError_t launch_qgemm(const QgemmArgs &a, const float *x, int64_t x_stride, int pro,
                         const float *gamma, const float *beta, float eps, hipStream_t s)
@@ -1607,7 +1354,17 @@ hipError_t launch_qgemm(const QgemmArgs &a, const float *x, int64_t x_stride, in
     const unsigned mp = (unsigned)((a.M + 15) / 16 * 16);
     int ipt = (K / 8 + 255) / 256;
 #define SMX_QPREP(KN) hipLaunchKernelGGL(KN, dim3(mp), dim3(256), 0, s, x, x_stride, a.M, K, pro, gamma, beta, eps, (uint8_t *)a.xp)
+#define SMX_QPREPT(P, S) hipLaunchKernelGGL((k_qprep_tokens<P, S>), dim3(mp / 4), dim3(256), 0, s, x, x_stride, a.M, K, gamma, beta, eps, (uint8_t *)a.xp)
     if (!x) ipt = -1;   // the parts are already in a.xp (written by the producing kernel)
+    if (x && a.M > 16) {
+        const int kind = qgemm_sums_kind(a.w, a.M);
+#define SMX_QPREPP(P) do { if (kind == 0) SMX_QPREPT(P, 0); else if (kind == 1) SMX_QPREPT(P, 1); else SMX_QPREPT(P, 2); } while (0)
+        if (pro == PRO_NONE) SMX_QPREPP(PRO_NONE);
+        else if (pro == PRO_RMS) SMX_QPREPP(PRO_RMS);
+        else SMX_QPREPP(PRO_LN);
+#undef SMX_QPREPP
+        ipt = -1;
+    }
     switch (ipt) {
     case -1: break;
     case 1: SMX_QPREP(k_qprep<1>); break;
@@ -1617,8 +1374,10 @@ hipError_t launch_qgemm(const QgemmArgs &a, const float *x, int64_t x_stride, in
     default: SMX_QPREP(k_qprep_long); break;
     }
 #undef SMX_QPREP
+#undef SMX_QPREPT
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+    if (qgemm_tiled(a.w, a.M)) return launch_qgemm_tile(a, s);
     switch (a.w.fmt) {
     case FMT_Q4_0: return launch_f<FMT_Q4_0>(a, s);
     case FMT_Q8_0: return launch_f<FMT_Q8_0>(a, s);

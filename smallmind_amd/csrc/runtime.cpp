@@ -97,7 +97,8 @@ int mat_alloc(Mat &m, int fmt, int64_t rows, int64_t cols)
         SMX_FAIL(SMX_EUNSUPPORTED, "matrix [%lld x %lld] exceeds the 4 GiB the kernels address", (long long)rows,
                  (long long)cols);
     SMX_HIP(hipMalloc((void **)&m.q, (size_t)(rows * nb * fmt_main_bytes(fmt))));
-    if (fmt_has_d(fmt)) SMX_HIP(hipMalloc((void **)&m.d, (size_t)(rows * nb * fmt_d_bytes(fmt))));
+    // (whole 32-bit words: an fp16 scale may be read with the aligned word that holds it)
+    if (fmt_has_d(fmt)) SMX_HIP(hipMalloc((void **)&m.d, (size_t)((rows * nb * fmt_d_bytes(fmt) + 3) & ~(int64_t)3)));
     m.fmt = fmt;
     m.rows = rows;
     m.cols = cols;
@@ -630,22 +631,27 @@ int run_tokens(const smx_model *m, TokBatch &B, int M, int ctx_stride, int head_
         } else {
             SMX_HIP(launch_qgemm(a, B.x, d, pro, L.d_attn_g, L.d_attn_b, c.norm_eps, s));
         }
-        // attention writes the O projection's activation parts directly (no k_qprep launch)
+        // attention writes the O projection's activation parts directly (no k_qprep launch), with
+        // their sub-block sums when that GEMM reads them (head_dim < 32: a sub-block would span
+        // two heads' workgroups, so the outputs go through k_qprep)
+        const XpSums sums{qgemm_sums_kind(L.o.view(), M), M};
+        const bool att_parts = !sums.kind || hd >= 32;
+        uint8_t *att_xp = att_parts ? B.xp2 : nullptr;
         if (run && n_blk > 0 && attention_prefill_supported(c.n_head, Hkv, hd)) {
             const PrefillBlocks pb{B.blk, B.kc, B.vc, B.pos, layer_off};
             SMX_HIP(launch_attention_prefill_blocks(B.q, m->nqkv, B.att, d, c.n_head, Hkv, hd, ctx_stride, n_blk, pb,
-                                                    s, B.xp2));
+                                                    s, att_xp, sums));
         } else if (run && attention_prefill_supported(c.n_head, Hkv, hd)) {
             for (int i = 0; i < n_run; i++) {
                 const PrefillRun &r = run[i];
                 const int cnt = r.count < 0 ? M : r.count;
                 SMX_HIP(launch_attention_prefill(B.q + (int64_t)r.row0 * m->nqkv, m->nqkv, r.kc + layer_off,
                                                  r.vc + layer_off, B.att + (int64_t)r.row0 * d, d, c.n_head, Hkv, hd,
-                                                 ctx_stride, r.p_first, cnt, s, B.xp2, r.row0));
+                                                 ctx_stride, r.p_first, cnt, s, att_xp, r.row0, sums));
             }
         } else
             SMX_HIP(launch_attention_tokens(B.q, m->nqkv, B.kc, B.vc, layer_off, B.att, d, c.n_head, Hkv, hd,
-                                            ctx_stride, B.pos, M, s, B.xp2));
+                                            ctx_stride, B.pos, M, s, att_xp, sums));
         QgemmArgs o{};
         o.w = L.o.view();
         o.xp = B.xp2;
@@ -659,7 +665,7 @@ int run_tokens(const smx_model *m, TokBatch &B, int M, int ctx_stride, int head_
             o.ngamma = L.d_ffn_g;
             o.nss = B.ss;
         }
-        SMX_HIP(launch_qgemm(o, nullptr, d, PRO_NONE, nullptr, nullptr, 0.0f, s));
+        SMX_HIP(launch_qgemm(o, att_parts ? nullptr : B.att, d, PRO_NONE, nullptr, nullptr, 0.0f, s));
         QgemmArgs g{};
         g.w = L.gu.view();
         g.xp = B.xp;
@@ -668,7 +674,12 @@ int run_tokens(const smx_model *m, TokBatch &B, int M, int ctx_stride, int head_
         g.y_stride = m->hidden;
         g.bias = L.d_bgu;
         g.epi = m->llama ? EPI_SILU : EPI_GELU;
-        g.yp = B.xp2;   // the down projection's activation parts
+        // the down projection's activation parts are written by the gate/up epilogue, unless it would
+        // need their sub-block sums too and only the tile kernel writes those
+        const int h_sums = qgemm_sums_kind(L.down.view(), M);
+        const bool h_parts = qgemm_tiled(L.gu.view(), M) || !h_sums;
+        if (h_parts) g.yp = B.xp2;
+        g.yp_sums = h_sums;
         if (fold) {
             g.rss = B.ss;
             g.rss_n = d / 16;
@@ -690,7 +701,7 @@ int run_tokens(const smx_model *m, TokBatch &B, int M, int ctx_stride, int head_
             dn.ngamma = m->layers[l + 1].d_attn_g;
             dn.nss = B.ss;
         }
-        SMX_HIP(launch_qgemm(dn, nullptr, m->hidden, PRO_NONE, nullptr, nullptr, 0.0f, s));
+        SMX_HIP(launch_qgemm(dn, h_parts ? nullptr : B.h, m->hidden, PRO_NONE, nullptr, nullptr, 0.0f, s));
     }
     if (head_from < M && fmt_dense(m->head.fmt)) {
         // an unquantized head: the fused GEMV (norm prologue per row), one pass per row
@@ -1081,7 +1092,8 @@ SMX_API int smx_weight_to_float32_host(const smx_weight *w, float *out)
 // of the process.  Host code never passes the array's name to a kernel or a copy (in host code
 // it names a host-side stand-in): it uses the per-device address from hipGetSymbolAddress.
 constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
-static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
+// (the limit counts the parts; their sub-block sums, 1/16 of the parts, lie behind them)
+static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes / 16 * 17];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -1130,7 +1142,7 @@ SMX_API int smx_weight_matmul_noalloc(const smx_weight *w, const float *act_dev,
         SMX_HIP(launch_gemv(a, m, st));
         return SMX_OK;
     }
-    const size_t need = qgemm_xp_bytes(m, k);
+    const size_t need = qgemm_parts_bytes(m, k);
     if (need > kNoAllocScratchBytes)
         SMX_FAIL(SMX_EINVAL, "smx_weight_matmul_noalloc: m=%d, k=%d needs %zu bytes of scratch; the limit is %zu "
                              "(ceil(m/16) * k/32 * 3072 bytes)", m, k, need, kNoAllocScratchBytes);

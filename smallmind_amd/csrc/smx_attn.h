@@ -29,13 +29,15 @@ struct AttnSmem {
 // sc: LDS scratch of at least n_pos floats.  All NT threads of the workgroup must call this.
 // U: positions per thread per P.V load batch (one batch = one round trip to memory).
 // With parts set, the output is written as activation parts of the next GEMM instead of out:
-// xp_store(parts, parts_nsb, parts_tok, parts_k0 + d, out[d]).
+// xp_store(parts, parts_nsb, parts_tok, parts_k0 + d, out[d]), and with sums.kind (HD >= 32) the sums
+// of their sub-blocks.
 template <int HD, int NT, int U = 8>
 __device__ __forceinline__ void attention_head(const float *__restrict__ qh, const float *__restrict__ K,
                                                const float *__restrict__ V, float *__restrict__ out,
                                                int n_pos, int ctx_stride, float *sc,
                                                AttnSmem<HD, NT> &sm, uint8_t *parts = nullptr,
-                                               int parts_nsb = 0, int parts_tok = 0, int parts_k0 = 0)
+                                               int parts_nsb = 0, int parts_tok = 0, int parts_k0 = 0,
+                                               XpSums sums = XpSums{})
 {
     constexpr int D4 = HD / 4;
     constexpr int NPL = NT / D4;
@@ -125,6 +127,13 @@ __device__ __forceinline__ void attention_head(const float *__restrict__ qh, con
             xp_store(parts, parts_nsb, parts_tok, k + 1, o.y);
             xp_store(parts, parts_nsb, parts_tok, k + 2, o.z);
             xp_store(parts, parts_nsb, parts_tok, k + 3, o.w);
+            if (HD >= 32 && sums.kind) {   // the 8 threads of a 32-dimension sub-block are neighbouring lanes
+                float q = (o.x + o.y) + (o.z + o.w);
+                q += dpp_mov<0xB1>(q);
+                q += dpp_mov<0x4E>(q);
+                const float other = dpp_mov<0x141>(q);
+                if ((tid & 7) == 0) xp_sums(parts, sums.kind, sums.M, parts_nsb, parts_tok, k >> 5, q, other);
+            }
         } else {
             ((float4 *)out)[tid] = o;
         }

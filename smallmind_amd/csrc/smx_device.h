@@ -161,6 +161,16 @@ __device__ __forceinline__ uint32_t bf16_rne(float f)
     return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// bf16 pair (round to nearest even), a in the low half
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b)
+{
+    const bf16x2 v = {(__bf16)a, (__bf16)b};
+    uint32_t r;
+    __builtin_memcpy(&r, &v, 4);
+    return r;
+}
+
 // Activation parts of the matrix-core GEMM (k_qgemm): f = hi + mid + lo, three bf16 values each
 // rounded to nearest even, stored for element k = 32 s + 8 g + 4 h + q of token m at
 // Xp[m / 16][s][part][g][m % 16] dword q, half h (2 bytes each; nsb = sub-blocks per token).
@@ -177,6 +187,30 @@ __device__ __forceinline__ void xp_store(uint8_t *xp, int nsb, int m, int k, flo
     *(uint16_t *)(b + 2048) = (uint16_t)bf16_rne(r2);
 }
 
+// Sums of the activations of sub-block s (32 elements) of token m, from which the GEMM over more
+// than 16 tokens takes its code-offset and min terms.  They are matrix-core operands, stored as
+// three bf16 parts behind the parts of all M tokens: kind 1 (one sum per sub-block)
+// [m / 16][s / 8][part][m % 16][s % 8], kind 2 (one per 16 elements) [m / 16][s / 8][part][half]
+// [m % 16][s % 8].
+__device__ __forceinline__ void xp_sums(uint8_t *xp, int kind, int M, int nsb, int m, int s, float first, float second)
+{
+    uint8_t *base = xp + (size_t)((M + 15) >> 4) * nsb * 3072u +
+                    ((size_t)(m >> 4) * (nsb >> 3) + (s >> 3)) * (768u * (uint32_t)kind) + (m & 15) * 16 + (s & 7) * 2;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        if (h && kind == 1) break;
+        const float f = kind == 1 ? first + second : h ? second : first;
+        const uint32_t hi = bf16_rne(f);
+        const float r1 = f - __uint_as_float(hi << 16);
+        const uint32_t mid = bf16_rne(r1);
+        const float r2 = r1 - __uint_as_float(mid << 16);
+        uint16_t *p = (uint16_t *)(base + 256 * h);
+        p[0] = (uint16_t)hi;
+        p[128 * kind] = (uint16_t)mid;
+        p[256 * kind] = (uint16_t)bf16_rne(r2);
+    }
+}
+
 // v_permlane32_swap_b32 (gfx950): lanes 32..63 of `a` trade places with lanes 0..31 of `b`;
 // .x is the new `a`, .y the new `b`.
 __device__ __forceinline__ float2 swap32(float a, float b)
@@ -190,6 +224,13 @@ __device__ __forceinline__ float2 swap16(float a, float b)
 {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
     return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// The value of lane l ^ 16 (the neighbouring 16-lane row of a 32-lane half).
+__device__ __forceinline__ float swap16_other(float v)
+{
+    const float2 p = swap16(v, v);
+    return (threadIdx.x & 16) ? p.x : p.y;
 }
 
 // Totals of R per-lane partials (R = 2 or 4) over the wave, transposed: row r's total ends up

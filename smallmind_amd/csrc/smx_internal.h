@@ -193,7 +193,8 @@ struct QgemmArgs {
     const float *bias;          // [rows] or nullptr (interleaved like the rows for EPI_SILU)
     int epi;                    // EPI_STORE / EPI_RESID / EPI_GELU / EPI_SILU / EPI_QKV
     // EPI_SILU / EPI_GELU: when set, the outputs go to yp as the activation parts of the next
-    // GEMM (qgemm_xp_bytes(M, width) bytes) instead of y
+    // GEMM (qgemm_xp_bytes(M, width) bytes) instead of y, with their sub-block sums of kind
+    // yp_sums (tile kernel only)
     uint8_t *yp;
     // EPI_QKV
     int d_model, kv_dim, head_dim, use_rope, ctx_stride;
@@ -215,9 +216,21 @@ struct QgemmArgs {
     const float *rss;
     int rss_n;
     float r_eps;
+    int yp_sums;
 };
-// Scratch bytes of the activation parts for M tokens of K elements.
+// Scratch bytes for M tokens of K elements: the activation parts, and the parts with the
+// sub-block sums behind them.
+size_t qgemm_parts_bytes(int M, int K);
 size_t qgemm_xp_bytes(int M, int K);
+// Whether the GEMM of M tokens with w runs on the tile kernel (k_qgemm_tile.hip), its number of 64 x 64
+// tiles, and which sub-block sums it reads (a kind of xp_sums, 0: none).
+bool qgemm_tiled(const WView &w, int M);
+int64_t qgemm_tiles(const WView &w, int M);
+int qgemm_sums_kind(const WView &w, int M);
+// Sub-block sums to write behind activation parts: their kind and the tokens of the whole batch.
+struct XpSums {
+    int kind = 0, M = 0;
+};
 // Prepares the parts of the (normalised, PRO_RMS / PRO_LN) activations into xp, then runs the
 // GEMM.  a.xp must point at qgemm_xp_bytes(a.M, cols) bytes of scratch.  With x == nullptr
 // (and PRO_NONE) a.xp already holds the parts, written by the producing kernel.
@@ -302,11 +315,12 @@ hipError_t launch_embed_tokens(const WView &tok, const WView *posw, const int32_
 // ([n_kv_head][hd][ctx_stride] / [n_kv_head][ctx_stride][hd]), out [M][out_stride].
 bool attention_prefill_supported(int n_head, int n_kv_head, int hd);
 // With out_parts set, the outputs are written as the activation parts of the next GEMM
-// (xp_store, token tok_off + t, element h*hd + d) instead of out.
+// (xp_store, token tok_off + t, element h*hd + d) instead of out; with sums.kind also their
+// sub-block sums.
 hipError_t launch_attention_prefill(const float *q, int q_stride, const float *kc, const float *vc, float *out,
                                     int out_stride, int n_head, int n_kv_head, int hd, int ctx_stride,
                                     int p_first, int M, hipStream_t s, uint8_t *out_parts = nullptr,
-                                    int tok_off = 0);
+                                    int tok_off = 0, XpSums sums = XpSums{});
 // Several sessions' runs of a token batch in one launch: workgroup b takes the rows
 // blk[2b] .. blk[2b] + blk[2b+1] - 1 of the batch (at most attention_prefill_block_rows rows, all
 // of one run), with that session's cache (kc_tok / vc_tok of its first row, plus layer_off) and
@@ -320,12 +334,13 @@ struct PrefillBlocks {
 int attention_prefill_block_rows(int n_head, int n_kv_head);
 hipError_t launch_attention_prefill_blocks(const float *q, int q_stride, float *out, int out_stride, int n_head,
                                            int n_kv_head, int hd, int ctx_stride, int n_blocks,
-                                           const PrefillBlocks &pb, hipStream_t s, uint8_t *out_parts = nullptr);
+                                           const PrefillBlocks &pb, hipStream_t s, uint8_t *out_parts = nullptr,
+                                           XpSums sums = XpSums{});
 hipError_t launch_attention_tokens(const float *q, int64_t q_stride, float *const *kc_tok,
                                    float *const *vc_tok, int64_t layer_off, float *out,
                                    int64_t out_stride, int n_head, int n_kv_head, int hd,
                                    int ctx_stride, const int32_t *tok_pos, int M, hipStream_t s,
-                                   uint8_t *out_parts = nullptr);
+                                   uint8_t *out_parts = nullptr, XpSums sums = XpSums{});   // sums: hd >= 32
 hipError_t launch_argmax_rows(const float *x, int n, int64_t stride, int M, int32_t *tok_next,
                               int32_t *tok_pos, int32_t *const *tok_arr, hipStream_t s);
 

@@ -145,6 +145,32 @@ def test_matmul_matrix_core_random_bytes(gpu, name):
         assert np.all(np.abs(Y[r] - ref) <= TIGHT * scale + 1e-30), r
 
 
+@pytest.mark.parametrize("name", [n for n in TYPES if n not in ("F16", "F32")])
+@pytest.mark.parametrize("m,N,K", [(1025, 4100, 256),     # 64 x 64 wave tiles; one super-block, one token in the last tile
+                                   (1100, 4160, 768),     # three super-blocks, whole row groups
+                                   (700, 3100, 512),      # two waves of 64 x 32
+                                   (517, 3600, 768),      # K split in two: 2 + 1 super-blocks
+                                   (1030, 200, 2304),     # K split in four: 3 + 3 + 3 + 0 super-blocks
+                                   (641, 70, 2048)])      # few rows, many tokens
+def test_matmul_tile_kernel_vs_float64(gpu, name, m, N, K):
+    """The tile kernel (long prompts) at the edges of its tiles and K splits, on random bytes (every
+    code, scale and min value, fp16 scales of any magnitude) and rows of very different size.  Bound
+    per output: fp32 accumulation of K products whose magnitudes sum to |w| . |x| (the sub-block
+    sums carry a code offset of at most 4 code widths); the GEMM bound of this file."""
+    import torch
+    qt = TYPES[name]
+    W = random_blocks(qt, N * K // O.BLOCK_ELEMS[qt], m + N)
+    X = np.random.default_rng(m + K).normal(0, 1, (m, K)).astype(np.float32)
+    X[m // 2] *= 1e-3
+    X[3] *= 1e4
+    Y = _dev(_gemv(qt, W, N, K, X, m=m)).double()
+    Wf = _dev(O.dequant(qt, W, N * K).reshape(N, K)).double()
+    Xd = _dev(X).double()
+    ref, scale = Xd @ Wf.t(), Xd.abs() @ Wf.abs().t()
+    worst = float(((Y - ref).abs() / (TIGHT * scale + 1e-30)).max())
+    assert worst <= 1.0, worst
+
+
 def test_fused_equals_dequant_then_matmul(gpu):
     """The reference's live equivalence check (ExpandedQuantizationTests.cs:229-250): fused
     quantized matmul == dequantize then fp32 matmul."""
