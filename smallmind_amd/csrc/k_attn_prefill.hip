@@ -1,5 +1,5 @@
 // k_attn_prefill.hip -- causal attention of a run of consecutive tokens of one session over its
-// KV cache, on the fp32 matrix cores (prefill chunks).
+// KV cache, on the bf16 matrix cores at fp32 accuracy (prefill chunks).
 //
 // Reference: MultiHeadAttention.Forward with T > 1 tokens over the KV cache
 // (MultiHeadAttention.cs:206-297): scores Q.K^T per head (ComputeAttentionScoresInPlace,
@@ -15,23 +15,34 @@
 // accumulates E.V.  The output is (sum_j e_j v_j) / sum, the reference's sum_j (e_j / sum) v_j
 // up to rounding.
 //
-// Work decomposition.  A workgroup owns 32 query rows of one KV head: 32 / G tokens x the G
-// query heads that share the KV head (GQA), so every K/V element it loads serves 32 rows.  Its
-// 8 waves split the keys in 16-key tiles (wave w: tiles w, w + 8, ...).  A wave loads one tile
-// at a time: without a register copy of the next tile the kernel takes 115 VGPRs and two
-// workgroups fit a CU, whose other waves hide the loads (prefill +0.6-1.3 % against one
-// workgroup per CU with the next tile's loads in flight).  Partial maxima, sums and
-// outputs of the 8 waves are combined through LDS in a fixed order.
+// What bounds it.  The fp32 matrix instructions run on the vector ALU's datapath: measured, two
+// vector instructions beside each v_mfma_f32_16x16x4_f32 take it from 33 to 49 cycles, whatever
+// the number of waves, so a kernel of fp32 products (50 % of the time) and FastExp (30 %) cannot
+// overlap them.  The bf16 products can (eight vector instructions per product almost free).  Q, K,
+// V and E therefore enter as three bf16 parts whose sum is the fp32 value (x = h + m + l), and a
+// product is the six leading part products hh, hm, mh, mm, hl, lh (what is left out is below
+// 2^-24 of |a| |b|), small ones first.  Then FastExp, at about 28 vector
+// instructions per score, bounds pass 2 about as much as the products do.
+// 2048 tokens at positions 2048 .. of 32 / 4 heads: 984 us with fp32 products, 502 now (464 GFLOP of
+// part products, 920 TFLOP/s; a large bf16 product of the library runs at 1190 here), error against
+// 64 bits 4.6e-7 -> 2.9e-7.
 //
-// Matrix cores: v_mfma_f32_16x16x4_f32 (fp32 products, fp32 accumulation).
-//   S^T = K . Q^T per (16-key tile, 16-row block): A = K (lane: key l % 16, dimension
-//   4j + l / 16 for step j), B = Q^T (lane: query l % 16, same dimension); D lane l holds keys
-//   4(l/16) + i of query l % 16.
-//   O = E . V per (16-row block, 16-dimension block): A = E (lane: query l % 16, key
-//   4(l/16) + j for step j -- exactly the scores lane l already holds), B = V (lane: dimension
-//   l % 16, key 4(l/16) + j); D lane l holds queries 4(l/16) + i of dimension l % 16.
-// K is dimension-major [HD][ctx_stride] and V position-major [ctx_stride][HD]: for one step,
-// lanes l % 16 read 16 consecutive floats of one row, four rows per load instruction.
+// Work decomposition.  A workgroup owns 32 RW query rows of one KV head: 32 RW / G tokens x the G
+// query heads that share the KV head (GQA); a wave owns 32 rows.  Tiles of 32 keys are split into
+// parts once per workgroup and shared through LDS (two slots: the next tile is loaded while the
+// current one is multiplied).  KW > 1: KW groups of RW waves take alternate tiles (short prompts,
+// where rows alone do not fill the chip); their maxima, sums and outputs are combined in LDS in a
+// fixed order.  The workgroups with most keys start first.
+//
+// Operands of v_mfma_f32_32x32x16_bf16 (lane l: li = l % 32, h = l / 32; 8 k-values per lane):
+//   S^T = K . Q^T: A = K (key li, dimensions 16 t + 8 h ..), B = Q^T (query li, same dimensions); D
+//   lane holds keys 8 (i / 4) + 4 h + i % 4 of query li in register i.
+//   O^T = V^T . E^T: B = E^T (query li): the 8 keys of k-step s are registers 8 s .. 8 s + 7 of the
+//   scores the lane already holds, i.e. keys 16 s + 8 q + 4 h + r; A = V^T (dimension li + 32 dt, the
+//   same keys).  D lane holds dimensions 32 dt + 8 (i / 4) + 4 h + i % 4 of query li.
+// Nothing is transposed, and maximum, sum and 1 / sum are the lane's own (two lanes per query).
+#include <type_traits>
+
 #include "smx_device.h"
 #include "smx_internal.h"
 
@@ -39,17 +50,415 @@ namespace smx {
 
 namespace {
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ f32x16 mma(uint4 a, uint4 b, f32x16 c)
+{
+    bf16x8 x, y;
+    __builtin_memcpy(&x, &a, 16);
+    __builtin_memcpy(&y, &b, 16);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
+}
+
+constexpr int kHD = 64;   // head dimension of this kernel
+constexpr int kKeys = 32; // keys per tile
+
+// Value of lane l ^ 32.
+__device__ __forceinline__ float half_other(float v)
+{
+    const float2 p = swap32(v, v);
+    return (threadIdx.x & 32) ? p.x : p.y;
+}
+
+// FastExp with the quotient formed as the IEEE division does for operands that need no scaling (1/4
+// <= den <= 700, |num| <= 700): reciprocal, one Newton step, quotient, residual correction.
+__device__ __forceinline__ float fastexp_q(float x)
+{
+    x = fmaxf(-87.3f, fminf(x, 88.7f));
+    const float x2 = x * x, h = x * 0.5f, q = x2 * 0.08333333f;
+    const float num = (1.0f + h) + q, den = (1.0f - h) + q;
+    float r = __builtin_amdgcn_rcpf(den);
+    r = __builtin_fmaf(__builtin_fmaf(-den, r, 1.0f), r, r);
+    const float t = num * r;
+    return __builtin_fmaf(__builtin_fmaf(-den, t, num), r, t);
+}
+
+// Three bf16 parts of eight values, as one operand each.
+__device__ __forceinline__ void split8(const float *v, uint4 *o)
+{
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) x[i] = v[i];
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        uint32_t w[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            w[k] = bf16_pair(x[2 * k], x[2 * k + 1]);
+            if (p < 2) {
+                x[2 * k] -= __uint_as_float(w[k] << 16);
+                x[2 * k + 1] -= __uint_as_float(w[k] & 0xFFFF0000u);
+            }
+        }
+        o[p] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
+// With pb.blk set (several sessions' runs of a batch in one launch), a workgroup's rows, cache
+// and first position come from the block table instead of the arguments: q, out and tok_off
+// move to the block's first batch row, and the block is a run of M <= TT tokens at t0 = 0.
+template <int RW, int KW>
+__global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
+    const float *__restrict__ q, int q_stride, const float *__restrict__ kc, const float *__restrict__ vc,
+    float *__restrict__ out, int out_stride, int n_head, int n_kv_head, int ctx_stride, int p_first, int M,
+    uint8_t *__restrict__ out_parts, int tok_off, XpSums sums, PrefillBlocks pb)
+{
+    constexpr int IT = 256 / (64 * RW);   // 8-element pieces of a K (V) tile per thread of a key group
+    struct Lds {
+        uint4 k[KW][2][4][3][2][kKeys];    // [slot][dimensions 16 t ..][part][half][key]
+        uint4 v[KW][2][3][2][2][kHD];      // [slot][part][k-step][half][dimension]
+        uint4 q[RW][4][3][64];             // the query parts: 48 registers a lane if they were held
+        float mx[KW][RW][kKeys], sum[KW][RW][kKeys];
+    };
+    struct Red {
+        float o[KW > 1 ? KW - 1 : 1][RW][2 * 16][64];
+    };
+    __shared__ __align__(16) uint8_t s_mem[sizeof(Lds)];
+    static_assert(KW == 1 || sizeof(Red) <= sizeof(uint4) * KW * 2 * 4 * 3 * 2 * kKeys * 2, "outputs reuse the tiles");
+    Lds &L = *(Lds *)s_mem;
+    Red &R = *(Red *)s_mem;
+    const int tid = threadIdx.x, lane = tid & 63, wv = wave_id();
+    const int rw = wv % RW, kg = wv / RW;
+    const int li = lane & 31, h = lane >> 5;
+    const int G = n_head / n_kv_head, TT = 32 * RW / G;
+    const int kvh = blockIdx.y;
+    int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * TT;   // longest rows first
+    if (pb.blk) {   // uniform over the workgroup
+        const int b = (int)gridDim.x - 1 - (int)blockIdx.x, r0 = pb.blk[2 * b];
+        M = pb.blk[2 * b + 1];
+        t0 = 0;
+        kc = pb.kc_tok[r0] + pb.layer_off;
+        vc = pb.vc_tok[r0] + pb.layer_off;
+        p_first = pb.pos[r0];
+        q += (int64_t)r0 * q_stride;
+        out += (int64_t)r0 * out_stride;
+        tok_off += r0;
+    }
+    // MultiHeadAttention.cs:682; a power of two, so scaling q instead of the scores changes no bit
+    const float scale = 1.0f / sqrtf((float)kHD);
+
+    // this lane's query: row 32 rw + li of the workgroup
+    const int row = 32 * rw + li;
+    const int tok = t0 + row / G, head = kvh * G + row % G;
+    const int npos = p_first + min(tok, M - 1) + 1;                      // keys the query sees
+    if (kg == 0) {
+        const float *qr = q + (int64_t)min(tok, M - 1) * q_stride + (int64_t)head * kHD;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = qr[16 * t + 8 * h + e] * scale;   // (scalar loads: q is 4-byte aligned)
+            uint4 p[3];
+            split8(x, p);
+#pragma unroll
+            for (int c = 0; c < 3; c++) L.q[rw][t][c][lane] = p[c];
+        }
+    }
+    const int n_max = p_first + min(t0 + TT, M);   // keys 0 .. n_max-1 are written cache entries
+    const int n_tiles = (n_max + kKeys - 1) / kKeys, n_it = (n_tiles + KW - 1) / KW;
+    // K and V of one KV head span less than 4 GiB: uniform base + 32-bit offsets
+    const float *K = kc + (int64_t)kvh * kHD * ctx_stride;
+    const float *V = vc + (int64_t)kvh * ctx_stride * kHD;
+    const uint32_t cs = (uint32_t)ctx_stride;
+    const int tg = tid - 64 * RW * kg;   // thread of its key group
+
+    // piece i of a K tile: 8 dimensions of one key; of a V tile: 8 keys (the order of a k-step's
+    // operand) of one dimension
+    float kr[IT][8], vr[IT][8];
+    // (keys are clamped into the cache row; a tile wholly inside it needs no per-key clamp)
+    const char *Kb = (const char *)K, *Vb = (const char *)V;
+    auto load_k = [&](int tile) {
+        const int t = min(tile, (ctx_stride - 1) / kKeys), last = ctx_stride - 1 - kKeys * t;
+#pragma unroll
+        for (int n = 0; n < IT; n++) {
+            const int i = tg + 64 * RW * n;
+            const uint32_t off = 4u * ((uint32_t)(8 * (i >> 5)) * cs + (uint32_t)min(i & 31, last));
+#pragma unroll
+            for (int e = 0; e < 8; e++) kr[n][e] = *(const float *)(Kb + 4u * ((uint32_t)e * cs + (uint32_t)(kKeys * t)) + off);
+        }
+    };
+    auto store_k = [&](int slot) {
+#pragma unroll
+        for (int n = 0; n < IT; n++) {
+            const int i = tg + 64 * RW * n, dg = i >> 5;
+            uint4 p[3];
+            split8(kr[n], p);
+#pragma unroll
+            for (int c = 0; c < 3; c++) L.k[kg][slot][dg >> 1][c][dg & 1][i & 31] = p[c];
+        }
+    };
+    auto load_v = [&](int tile) {
+        const int t = min(tile, (ctx_stride - 1) / kKeys);
+        const char *b = Vb + 4u * (uint32_t)(kKeys * t * kHD);
+#pragma unroll
+        for (int n = 0; n < IT; n++) {
+            const int i = tg + 64 * RW * n, sh = i >> 6;
+            const int k0 = 16 * (sh >> 1) + 4 * (sh & 1);
+            if (kKeys * (t + 1) <= ctx_stride) {   // uniform
+                const uint32_t off = 4u * (uint32_t)(k0 * kHD + (i & 63));
+#pragma unroll
+                for (int e = 0; e < 8; e++) vr[n][e] = *(const float *)(b + off + 4 * kHD * (8 * (e >> 2) + (e & 3)));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const int key = min(k0 + 8 * (e >> 2) + (e & 3), ctx_stride - 1 - kKeys * t);
+                    vr[n][e] = *(const float *)(b + 4u * (uint32_t)(key * kHD + (i & 63)));
+                }
+            }
+        }
+    };
+    auto store_v = [&](int slot, int tile, auto tail) {
+#pragma unroll
+        for (int n = 0; n < IT; n++) {
+            const int i = tg + 64 * RW * n, sh = i >> 6;
+            // V rows past the written cache entries may hold anything: zero them (0 * NaN)
+#pragma unroll
+            for (int e = 0; decltype(tail)::value && e < 8; e++) {
+                const int key = kKeys * tile + 16 * (sh >> 1) + 8 * (e >> 2) + 4 * (sh & 1) + (e & 3);
+                vr[n][e] = key < n_max ? vr[n][e] : 0.0f;
+            }
+            uint4 p[3];
+            split8(vr[n], p);
+#pragma unroll
+            for (int c = 0; c < 3; c++) L.v[kg][slot][c][sh >> 1][sh & 1][i & 63] = p[c];
+        }
+    };
+    // scores of one tile: s[i] = key 8 (i / 4) + 4 h + i % 4 of the tile, query li
+    auto scores = [&](int slot, f32x16 &s) {
+        int z = 0;   // opaque: the query parts are read at each use and not kept in registers
+        asm volatile("" : "+s"(z));
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const uint4 kh = L.k[kg][slot][t][0][h][li], km = L.k[kg][slot][t][1][h][li], kl = L.k[kg][slot][t][2][h][li];
+            const uint4 qh = L.q[rw + z][t][0][lane], qm = L.q[rw + z][t][1][lane], ql = L.q[rw + z][t][2][lane];
+            s = mma(kl, qh, s);
+            s = mma(kh, ql, s);
+            s = mma(km, qm, s);
+            s = mma(km, qh, s);
+            s = mma(kh, qm, s);
+            s = mma(kh, qh, s);
+        }
+    };
+
+    // Iterations whose tiles (of every key group) hold only keys that all of the workgroup's queries
+    // see need no mask.  Tile indices past the last one load clamped keys into slots that are masked
+    // or not read.
+    const int it_full = min(n_it, max(0, (p_first + min(t0, M - 1) + 1) / kKeys - (KW - 1)) / KW);
+    auto seen = [&](int tile, int i) { return kKeys * tile + 8 * (i >> 2) + 4 * h + (i & 3) < npos; };
+
+    // ---- pass 1: row maxima -----------------------------------------------------------------
+    // (the next tile is split under the current one's products, the one after it is in flight)
+    float mx = -INFINITY;
+    load_k(kg);
+    store_k(0);
+    load_k(kg + KW);
+    __syncthreads();
+    auto pass1 = [&](int it, auto masked) {
+        const int tile = kg + KW * it;
+        f32x16 s;
+        scores(it & 1, s);
+        store_k((it + 1) & 1);
+        load_k(tile + 2 * KW);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            if constexpr (decltype(masked)::value) mx = fmaxf(mx, seen(tile, i) ? s[i] : -INFINITY);
+            else mx = fmaxf(mx, s[i]);
+        }
+        __syncthreads();
+    };
+    int it1 = 0;
+    for (; it1 < it_full; it1++) pass1(it1, std::false_type{});
+    for (; it1 < n_it; it1++) pass1(it1, std::true_type{});
+    mx = fmaxf(mx, half_other(mx));
+    if constexpr (KW > 1) {
+        if (h == 0) L.mx[kg][rw][li] = mx;
+    }
+
+    // ---- pass 2: exponentials, sums and E.V --------------------------------------------------
+    // Iteration it multiplies the scores of tile it + 1 while it exponentiates those of tile it, then
+    // E.V of tile it while the next tiles are split into the slots read last in iteration it - 1.
+    load_k(kg);
+    load_v(kg);
+    store_k(0);
+    store_v(0, kg, std::true_type{});
+    load_k(kg + KW);
+    load_v(kg + KW);
+    __syncthreads();
+    f32x16 s0, s1;
+    scores(0, s0);
+    store_k(1);
+    load_k(kg + 2 * KW);
+    if constexpr (KW > 1) {
+        mx = L.mx[0][rw][li];
+#pragma unroll
+        for (int k = 1; k < KW; k++) mx = fmaxf(mx, L.mx[k][rw][li]);
+    }
+    __syncthreads();
+    float sum = 0.0f;
+    f32x16 oh[2];   // dimensions 32 dt ..
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) oh[dt][i] = 0.0f;
+    // s: scores of tile it in, sn: of tile it + 1 out
+    auto pass2 = [&](int it, f32x16 &s, f32x16 &sn, auto masked, auto tail) {
+        const int tile = kg + KW * it, slot = it & 1;
+        scores(slot ^ 1, sn);
+        float sc[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            sc[i] = fastexp_q(s[i] - mx);
+            if constexpr (decltype(masked)::value) sc[i] = seen(tile, i) ? sc[i] : 0.0f;
+        }
+        float ts[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) ts[i] = sc[i] + sc[8 + i];
+        sum += ((ts[0] + ts[1]) + (ts[2] + ts[3])) + ((ts[4] + ts[5]) + (ts[6] + ts[7]));
+        uint4 ep[2][3];
+        split8(sc, ep[0]);
+        split8(sc + 8, ep[1]);
+        // the tile's products are summed by themselves and added to the output once, so that the
+        // output takes one rounding per tile and not one per part product
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++) {
+            f32x16 d;
+#pragma unroll
+            for (int i = 0; i < 16; i++) d[i] = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                uint4 vp[3];
+#pragma unroll
+                for (int p = 0; p < 3; p++) vp[p] = L.v[kg][slot][p][ks][h][32 * dt + li];
+                d = mma(vp[2], ep[ks][0], d);
+                d = mma(vp[0], ep[ks][2], d);
+                d = mma(vp[1], ep[ks][1], d);
+                d = mma(vp[1], ep[ks][0], d);
+                d = mma(vp[0], ep[ks][1], d);
+                d = mma(vp[0], ep[ks][0], d);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) oh[dt][i] += d[i];
+        }
+        store_k(slot);
+        store_v(slot ^ 1, tile + KW, tail);
+        load_k(tile + 3 * KW);
+        load_v(tile + 2 * KW);
+        __syncthreads();
+    };
+    // pairs of iterations, so that the two score registers trade places without copies
+    int it = 0;
+    for (; it + 2 < it_full; it += 2) {
+        pass2(it, s0, s1, std::false_type{}, std::false_type{});
+        pass2(it + 1, s1, s0, std::false_type{}, std::false_type{});
+    }
+    for (; it < n_it; it += 2) {
+        pass2(it, s0, s1, std::true_type{}, std::true_type{});
+        if (it + 1 < n_it) pass2(it + 1, s1, s0, std::true_type{}, std::true_type{});
+    }
+    sum += half_other(sum);
+    if constexpr (KW > 1) {   // the key groups' sums and outputs, added in order by group 0
+        if (h == 0) L.sum[kg][rw][li] = sum;
+        if (kg > 0) {
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) R.o[kg - 1][rw][16 * dt + i][lane] = oh[dt][i];
+        }
+        __syncthreads();
+        if (kg > 0) return;
+        sum = L.sum[0][rw][li];
+#pragma unroll
+        for (int k = 1; k < KW; k++) {
+            sum += L.sum[k][rw][li];
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) oh[dt][i] += R.o[k - 1][rw][16 * dt + i][lane];
+        }
+    }
+    const float inv = 1.0f / sum;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) oh[dt][i] *= inv;
+    const bool live = tok < M;
+    if (!out_parts) {
+        if (!live) return;
+        float *o = out + (int64_t)tok * out_stride + (int64_t)head * kHD + 4 * h;
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                *(float4 *)(o + 32 * dt + 8 * g) = make_float4(oh[dt][4 * g], oh[dt][4 * g + 1], oh[dt][4 * g + 2], oh[dt][4 * g + 3]);
+        return;
+    }
+    // Activation parts of the O projection: the lanes l and l ^ 32 hold elements r and r + 4 of each
+    // group of 8, i.e. the two halves of the pairs a part stores; lane half h stores groups h, h + 2.
+    const int nsb = n_head * kHD / 32, m = tok_off + tok;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++) {
+        const int sb = head * (kHD / 32) + dt;
+        uint8_t *p = out_parts + ((size_t)(m >> 4) * nsb + sb) * 3072u + (m & 15) * 16;
+#pragma unroll
+        for (int gg = 0; gg < 2; gg++) {
+            float lo[4], hi[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float2 e = swap32(oh[dt][8 * gg + r], oh[dt][8 * gg + r]);           // group 2 gg
+                const float2 f = swap32(oh[dt][8 * gg + 4 + r], oh[dt][8 * gg + 4 + r]);   // group 2 gg + 1
+                lo[r] = h ? f.x : e.x;
+                hi[r] = h ? f.y : e.y;
+            }
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                uint32_t w[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    w[r] = bf16_pair(lo[r], hi[r]);
+                    lo[r] -= __uint_as_float(w[r] << 16);
+                    hi[r] -= __uint_as_float(w[r] & 0xFFFF0000u);
+                }
+                if (live) *(uint4 *)(p + 1024 * c + 256 * (2 * gg + h)) = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+        if (sums.kind) {
+            float a = 0.0f, b = 0.0f;   // dimensions 0..15 and 16..31 of the sub-block
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                a += oh[dt][i];
+                b += oh[dt][8 + i];
+            }
+            a += half_other(a);
+            b += half_other(b);
+            if (live && h == 0) xp_sums(out_parts, sums.kind, sums.M, nsb, m, sb, a, b);
+        }
+    }
+}
+
+// ---- few rows ------------------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c)
+__device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-constexpr int kHD = 64;          // head dimension of this kernel
-constexpr int kRows = 32;        // query rows per workgroup (two 16-row blocks)
-constexpr int kWaves = 8;
-constexpr int kPitch = kHD + 4;  // LDS row pitch of the partial outputs (conflict-free writes)
+constexpr int kFewRows = 32;         // query rows per workgroup (two 16-row blocks)
+constexpr int kFewWaves = 8;
+constexpr int kFewPitch = kHD + 4;   // LDS row pitch of the partial outputs (conflict-free writes)
 
 // Maximum / sum over the four 16-lane rows (lanes l, l^16, l^32, l^48), the same bits in all.
 __device__ __forceinline__ float rows_max(float v)
@@ -67,19 +476,26 @@ __device__ __forceinline__ float rows_sum(float v)
     return p.x + p.y;
 }
 
-// With pb.blk set (several sessions' runs of a batch in one launch), workgroup b's rows, cache
-// and first position come from the block table instead of the arguments: q, out and tok_off
-// move to the block's first batch row, and the block is a run of M <= TT tokens at t0 = 0.
-__global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
+// The same attention for few rows, where the time is the chain of keys of one workgroup and not
+// the products: 32 query rows per workgroup, whose 8 waves split the keys in 16-key tiles (wave w:
+// tiles w, w + 8, ...), fp32 products (v_mfma_f32_16x16x4_f32), the same two passes; partial
+// maxima, sums and outputs of the waves are combined through LDS in a fixed order.
+//   S^T = K . Q^T per (16-key tile, 16-row block): A = K (lane: key l % 16, dimension
+//   4j + l / 16 for step j), B = Q^T (lane: query l % 16, same dimension); D lane l holds keys
+//   4(l/16) + i of query l % 16.
+//   O = E . V per (16-row block, 16-dimension block): A = E (lane: query l % 16, key
+//   4(l/16) + j for step j -- exactly the scores lane l already holds), B = V (lane: dimension
+//   l % 16, key 4(l/16) + j); D lane l holds queries 4(l/16) + i of dimension l % 16.
+__global__ __launch_bounds__(kFewWaves * 64) void k_attn_prefill_few(
     const float *__restrict__ q, int q_stride, const float *__restrict__ kc, const float *__restrict__ vc,
     float *__restrict__ out, int out_stride, int n_head, int n_kv_head, int ctx_stride, int p_first, int M,
     uint8_t *__restrict__ out_parts, int tok_off, XpSums sums, PrefillBlocks pb)
 {
-    extern __shared__ float s_out[];          // [kWaves][kRows][kPitch]
-    __shared__ float s_max[kWaves][kRows], s_sum[kWaves][kRows], s_inv[kRows];
+    extern __shared__ float s_out[];          // [kFewWaves][kFewRows][kFewPitch]
+    __shared__ float s_max[kFewWaves][kFewRows], s_sum[kFewWaves][kFewRows], s_inv[kFewRows];
     const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
     const int li = lane & 15, g = lane >> 4;
-    const int G = n_head / n_kv_head, TT = kRows / G;
+    const int G = n_head / n_kv_head, TT = kFewRows / G;
     const int kvh = blockIdx.y;
     int t0 = blockIdx.x * TT;
     if (pb.blk) {   // uniform over the workgroup
@@ -132,8 +548,8 @@ __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
         f32x4 a0 = {0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
 #pragma unroll
         for (int j = 0; j < 16; j++) {
-            a0 = mma(kv[j], qv[0][j], a0);
-            a1 = mma(kv[j], qv[1][j], a1);
+            a0 = mma4(kv[j], qv[0][j], a0);
+            a1 = mma4(kv[j], qv[1][j], a1);
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -147,7 +563,7 @@ __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
     {
         float kv[16];
         int ti = w;
-        for (; ti < n_tiles; ti += kWaves) {
+        for (; ti < n_tiles; ti += kFewWaves) {
             load_k(ti, kv);
             float s[2][4];
             scores(kv, s);
@@ -168,7 +584,7 @@ __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
     for (int rb = 0; rb < 2; rb++) {
         float m = s_max[0][16 * rb + li];
 #pragma unroll
-        for (int v = 1; v < kWaves; v++) m = fmaxf(m, s_max[v][16 * rb + li]);
+        for (int v = 1; v < kFewWaves; v++) m = fmaxf(m, s_max[v][16 * rb + li]);
         mx[rb] = m;
     }
 
@@ -182,7 +598,7 @@ __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
     {
         float kv[16], vv[4][4];
         int ti = w;
-        for (; ti < n_tiles; ti += kWaves) {
+        for (; ti < n_tiles; ti += kFewWaves) {
             load_k(ti, kv);
             load_v(ti, vv);
             float s[2][4];
@@ -203,8 +619,8 @@ __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
 #pragma unroll
                 for (int mb = 0; mb < 4; mb++) {
                     const float vz = ok ? vv[j][mb] : 0.0f;
-                    o[0][mb] = mma(s[0][j], vz, o[0][mb]);
-                    o[1][mb] = mma(s[1][j], vz, o[1][mb]);
+                    o[0][mb] = mma4(s[0][j], vz, o[0][mb]);
+                    o[1][mb] = mma4(s[1][j], vz, o[1][mb]);
                 }
             }
 
@@ -219,22 +635,22 @@ __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
         for (int mb = 0; mb < 4; mb++)
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                s_out[(w * kRows + 16 * rb + 4 * g + i) * kPitch + 16 * mb + li] = o[rb][mb][i];
+                s_out[(w * kFewRows + 16 * rb + 4 * g + i) * kFewPitch + 16 * mb + li] = o[rb][mb][i];
     }
     __syncthreads();
-    if (tid < kRows) {
+    if (tid < kFewRows) {
         float sm = s_sum[0][tid];
 #pragma unroll
-        for (int v = 1; v < kWaves; v++) sm += s_sum[v][tid];
+        for (int v = 1; v < kFewWaves; v++) sm += s_sum[v][tid];
         s_inv[tid] = 1.0f / sm;
     }
     __syncthreads();
     // combine: thread -> (row r, 4 dimensions)
     const int r = tid >> 4, d4 = (tid & 15) * 4;
-    float4 acc = *(const float4 *)&s_out[r * kPitch + d4];
+    float4 acc = *(const float4 *)&s_out[r * kFewPitch + d4];
 #pragma unroll
-    for (int v = 1; v < kWaves; v++) {
-        const float4 p = *(const float4 *)&s_out[(v * kRows + r) * kPitch + d4];
+    for (int v = 1; v < kFewWaves; v++) {
+        const float4 p = *(const float4 *)&s_out[(v * kFewRows + r) * kFewPitch + d4];
         acc.x += p.x; acc.y += p.y; acc.z += p.z; acc.w += p.w;
     }
     const int t = t0 + r / G;
@@ -261,13 +677,47 @@ __global__ __launch_bounds__(kWaves * 64) void k_attn_prefill(
     }
 }
 
+constexpr int kRW = 4, kKW = 2;      // k_attn_prefill: 128 rows per workgroup, keys split in two
+
+// Whether `rows` query rows (tokens x heads) fill the chip as 128-row workgroups.  Below about 100 of
+// them the chain of keys of each counts and the 32-row kernel is faster.  Measured (us, 32-row /
+// 128-row): 32 / 4 heads, 511 tokens (128 workgroups) 51 / 41, 32 / 8 heads, 700 tokens at 500 .. (176)
+// 147 / 90; 32 / 32 heads, 255 tokens (64) 21 / 28; 32 / 4 heads, 40 tokens at 1000 .. (10) 49 / 77.
+bool many_rows(int64_t rows) { return rows >= 100 * 32 * kRW; }
+
 }  // namespace
 
 bool attention_prefill_supported(int n_head, int n_kv_head, int hd)
 {
     if (hd != kHD || n_kv_head <= 0 || n_head % n_kv_head) return false;
     const int G = n_head / n_kv_head;
-    return G <= kRows && kRows % G == 0;
+    return G <= 32 && 32 % G == 0;
+}
+
+template <bool MANY>
+hipError_t launch_prefill(unsigned blocks, const float *q, int q_stride, const float *kc, const float *vc, float *out,
+                          int out_stride, int n_head, int n_kv_head, int ctx_stride, int p_first, int M, hipStream_t s,
+                          uint8_t *out_parts, int tok_off, XpSums sums, const PrefillBlocks &pb)
+{
+    const dim3 grid(blocks, (unsigned)n_kv_head);
+    if constexpr (MANY) {
+        hipLaunchKernelGGL((k_attn_prefill<kRW, kKW>), grid, dim3(64 * kRW * kKW), 0, s, q, q_stride, kc, vc, out,
+                           out_stride, n_head, n_kv_head, ctx_stride, p_first, M, out_parts, tok_off, sums, pb);
+    } else {
+        const size_t lds = (size_t)kFewWaves * kFewRows * kFewPitch * 4;
+        const hipError_t e = hipFuncSetAttribute((const void *)k_attn_prefill_few,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_attn_prefill_few, grid, dim3(kFewWaves * 64), lds, s, q, q_stride, kc, vc, out, out_stride,
+                           n_head, n_kv_head, ctx_stride, p_first, M, out_parts, tok_off, sums, pb);
+    }
+    return hipGetLastError();
+}
+
+// tokens per workgroup of the kernel that runs `tokens` tokens
+int attention_prefill_block_rows(int n_head, int n_kv_head, int tokens)
+{
+    return (many_rows((int64_t)tokens * n_head) ? 32 * kRW : kFewRows) / (n_head / n_kv_head);
 }
 
 hipError_t launch_attention_prefill(const float *q, int q_stride, const float *kc, const float *vc, float *out,
@@ -278,34 +728,28 @@ hipError_t launch_attention_prefill(const float *q, int q_stride, const float *k
     if (!attention_prefill_supported(n_head, n_kv_head, hd) || M <= 0 || p_first < 0 || ((n_head * hd) & 31) ||
         p_first + M > ctx_stride || (q_stride & 3) || (out_stride & 3) || tok_off < 0)
         return hipErrorInvalidValue;
-    const size_t lds = (size_t)kWaves * kRows * kPitch * 4;
-    const hipError_t e = hipFuncSetAttribute((const void *)k_attn_prefill,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    const int TT = kRows / (n_head / n_kv_head);
-    const dim3 grid((unsigned)((M + TT - 1) / TT), (unsigned)n_kv_head);
-    hipLaunchKernelGGL(k_attn_prefill, grid, dim3(kWaves * 64), lds, s, q, q_stride, kc, vc, out, out_stride,
-                       n_head, n_kv_head, ctx_stride, p_first, M, out_parts, tok_off, sums, PrefillBlocks{});
-    return hipGetLastError();
+    const int TT = attention_prefill_block_rows(n_head, n_kv_head, M);
+    const unsigned blocks = (unsigned)((M + TT - 1) / TT);
+    return many_rows((int64_t)M * n_head)
+               ? launch_prefill<true>(blocks, q, q_stride, kc, vc, out, out_stride, n_head, n_kv_head, ctx_stride, p_first,
+                                      M, s, out_parts, tok_off, sums, PrefillBlocks{})
+               : launch_prefill<false>(blocks, q, q_stride, kc, vc, out, out_stride, n_head, n_kv_head, ctx_stride, p_first,
+                                       M, s, out_parts, tok_off, sums, PrefillBlocks{});
 }
 
-int attention_prefill_block_rows(int n_head, int n_kv_head) { return kRows / (n_head / n_kv_head); }
-
 hipError_t launch_attention_prefill_blocks(const float *q, int q_stride, float *out, int out_stride, int n_head,
-                                           int n_kv_head, int hd, int ctx_stride, int n_blocks,
+                                           int n_kv_head, int hd, int ctx_stride, int n_blocks, int tokens,
                                            const PrefillBlocks &pb, hipStream_t s, uint8_t *out_parts, XpSums sums)
 {
-    if (!attention_prefill_supported(n_head, n_kv_head, hd) || n_blocks <= 0 || !pb.blk || !pb.kc_tok ||
-        !pb.vc_tok || !pb.pos || ((n_head * hd) & 31) || (q_stride & 3) || (out_stride & 3))
+    if (!attention_prefill_supported(n_head, n_kv_head, hd) || n_blocks <= 0 || tokens < n_blocks || !pb.blk ||
+        !pb.kc_tok || !pb.vc_tok || !pb.pos || ((n_head * hd) & 31) || (q_stride & 3) || (out_stride & 3))
         return hipErrorInvalidValue;
-    const size_t lds = (size_t)kWaves * kRows * kPitch * 4;
-    const hipError_t e = hipFuncSetAttribute((const void *)k_attn_prefill,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    const dim3 grid((unsigned)n_blocks, (unsigned)n_kv_head);
-    hipLaunchKernelGGL(k_attn_prefill, grid, dim3(kWaves * 64), lds, s, q, q_stride, nullptr, nullptr, out,
-                       out_stride, n_head, n_kv_head, ctx_stride, 0, 0, out_parts, 0, sums, pb);
-    return hipGetLastError();
+    const unsigned blocks = (unsigned)n_blocks;
+    return many_rows((int64_t)tokens * n_head)
+               ? launch_prefill<true>(blocks, q, q_stride, nullptr, nullptr, out, out_stride, n_head, n_kv_head, ctx_stride,
+                                      0, 0, s, out_parts, 0, sums, pb)
+               : launch_prefill<false>(blocks, q, q_stride, nullptr, nullptr, out, out_stride, n_head, n_kv_head, ctx_stride,
+                                       0, 0, s, out_parts, 0, sums, pb);
 }
 
 }  // namespace smx

@@ -639,8 +639,8 @@ int run_tokens(const smx_model *m, TokBatch &B, int M, int ctx_stride, int head_
         uint8_t *att_xp = att_parts ? B.xp2 : nullptr;
         if (run && n_blk > 0 && attention_prefill_supported(c.n_head, Hkv, hd)) {
             const PrefillBlocks pb{B.blk, B.kc, B.vc, B.pos, layer_off};
-            SMX_HIP(launch_attention_prefill_blocks(B.q, m->nqkv, B.att, d, c.n_head, Hkv, hd, ctx_stride, n_blk, pb,
-                                                    s, att_xp, sums));
+            SMX_HIP(launch_attention_prefill_blocks(B.q, m->nqkv, B.att, d, c.n_head, Hkv, hd, ctx_stride, n_blk, M,
+                                                    pb, s, att_xp, sums));
         } else if (run && attention_prefill_supported(c.n_head, Hkv, hd)) {
             for (int i = 0; i < n_run; i++) {
                 const PrefillRun &r = run[i];
@@ -812,13 +812,13 @@ int prefill_sessions(smx_model *m, TokBatch &P, smx_session *const *sessions, in
     // launch per layer for all sessions of the chunk instead of one per run
     const smx_model_config &c = m->cfg;
     const bool blocks = attention_prefill_supported(c.n_head, c.n_kv_head, m->hd);
-    const int TB = blocks ? attention_prefill_block_rows(c.n_head, c.n_kv_head) : 1;
     std::vector<int32_t> blk((size_t)cap * 2);
     int M = 0;
     auto flush = [&]() -> int {
         if (M == 0) return SMX_OK;
         int nb = 0;
         if (blocks && runs.size() > 1) {
+            const int TB = attention_prefill_block_rows(c.n_head, c.n_kv_head, M);
             for (const PrefillRun &r : runs)
                 for (int t = 0; t < r.count; t += TB) {
                     blk[(size_t)(2 * nb)] = r.row0 + t;

@@ -139,6 +139,35 @@ def test_attention_prefill_vs_oracle(gpu, H, Hkv, p0, n):
     assert rel_err(got, ref) < 2e-5
 
 
+@pytest.mark.parametrize("H,Hkv,p0,n", [(32, 4, 0, 401),     # 128-row workgroups of 16 tokens, the last with one
+                                        (32, 32, 37, 420),   # 128 tokens per workgroup, ragged; keys split 8 + 7 tiles
+                                        (32, 1, 95, 405),    # 4 tokens per workgroup
+                                        (12, 12, 5, 1070)])
+def test_attention_prefill_many_rows_vs_float64(gpu, H, Hkv, p0, n):
+    """The 128-row kernel (12800 query rows and more): against float64 with the same FastExp, cache
+    entries past the last token NaN, q at an address that is only 4-byte aligned.  Bound: the op
+    bound of this file."""
+    import torch
+    from smallmind_amd.quantization import attention_prefill
+    hd, ctx, kl = 64, p0 + n + 3, p0 + n
+    g = torch.Generator("cuda").manual_seed(H * 7 + n)
+    q = torch.randn(n * H * hd + 1, device="cuda", generator=g)[1:].reshape(n, H, hd)
+    k = torch.randn(Hkv, hd, ctx, device="cuda", generator=g)
+    v = torch.randn(Hkv, ctx, hd, device="cuda", generator=g)
+    k[:, :, kl:] = float("nan")
+    v[:, kl:] = float("nan")
+    got = attention_prefill(q, k, v, H, Hkv, hd, ctx, p0, n).reshape(n, H, hd).double()
+    seen = torch.arange(kl, device="cuda")[None] <= p0 + torch.arange(n, device="cuda")[:, None]
+    for h in range(H):
+        kv = h // (H // Hkv)
+        s = (q[:, h].double() @ k[kv, :, :kl].double() / 8.0).masked_fill(~seen, -float("inf"))
+        x = (s - s.amax(1, keepdim=True)).clamp(-87.3, 88.7)
+        e = torch.where(seen, (1 + x * 0.5 + x * x * 0.08333333) / (1 - x * 0.5 + x * x * 0.08333333), 0.0)
+        ref = e @ v[kv, :kl].double() / e.sum(1, keepdim=True)
+        assert torch.isfinite(got[:, h]).all()
+        assert float((got[:, h] - ref).abs().max() / ref.abs().max()) < 2e-5
+
+
 def test_silu_mul_gelu(gpu):
     from smallmind_amd.quantization import gelu, silu_mul
     rng = np.random.default_rng(1)
