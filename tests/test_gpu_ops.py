@@ -228,6 +228,82 @@ def test_sample_vs_oracle(gpu, n, opts):
             assert tok == otok, (u, tok, otok)
 
 
+def _sample64(l, ctx, temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, repetition_penalty=1.0, frequency_penalty=0.0,
+              repetition_window=0):
+    """Float32 logits stages, float64 probabilities: (probabilities, whether a cutoff lies within rounding)."""
+    l, f = l.copy(), np.float32
+    w = ctx[len(ctx) - min(len(ctx), repetition_window or 256):]
+    for t in np.unique(w):
+        if repetition_penalty != 1.0:
+            l[t] = l[t] / f(repetition_penalty) if l[t] > 0 else l[t] * f(repetition_penalty)
+        l[t] -= f(np.sum(w == t)) * f(frequency_penalty)
+    l = l * (f(1) / f(temperature))
+    if 0 < top_k < len(l):
+        l = np.where(l >= np.sort(l)[len(l) - top_k], l, f(-np.inf))
+    e = np.exp(l.astype(np.float64) - l.max())
+    p, near = e / e.sum(), False
+    if top_p < 1.0:
+        v, c = np.unique(p, return_counts=True)
+        cum = np.cumsum((v * c)[::-1])
+        near |= bool((np.abs(cum - top_p) < 1e-5).any())
+        p = np.where(p >= v[::-1][np.argmax(cum >= top_p)], p, 0.0)
+        p /= p.sum()
+    if min_p > 0.0:
+        near |= bool((np.abs(p / (p.max() * min_p) - 1) < 1e-5).any())
+        p = np.where(p < p.max() * min_p, 0.0, p)
+        p /= p.sum()
+    return p, near
+
+
+@pytest.mark.parametrize("n", [1, 63, 1025, 32000, 32768, 32769, 50257, 65536, 65537])
+@pytest.mark.parametrize("data", ["spread", "flat", "ties", "zeros", "masked"])
+def test_sample_paths_vs_float64(gpu, n, data):
+    """Values in LDS, in LDS and registers, and in memory; cutoffs found in the list of candidates and
+    outside of it (flat: more candidates than it holds; ties across the cutoff; fewer finite logits than
+    top-k; +0 and -0 at the cutoff).  Bound: sums of up to 65537 fp32 terms in a tree of depth 16 and
+    expf, 32 roundings of 2^-24 and the 2 ulp of expf on each side."""
+    from smallmind_amd.quantization import sample
+    rng = np.random.default_rng(n + len(data))
+    l = rng.normal(0, {"flat": 0.05}.get(data, 3.0), n).astype(np.float32)
+    if data == "ties":
+        l = np.round(l)
+    if data == "zeros":
+        l = np.where(rng.random(n) < 0.5, np.float32(0.0), np.float32(-0.0)) - (l > 1) * np.float32(1.0)
+        l[: n // 2] = -np.float32(0.0)
+    if data == "masked":
+        l[rng.permutation(n)[20:]] = -np.inf
+    ctx = rng.integers(0, n, 2500).astype(np.int32)
+    for kw in [dict(top_k=40, top_p=0.9, min_p=0.02, temperature=0.8, repetition_penalty=1.1),
+               dict(top_k=192), dict(top_k=193, top_p=0.5), dict(top_p=0.3), dict(top_p=0.95, frequency_penalty=0.1),
+               dict(min_p=0.1, repetition_penalty=1.2, repetition_window=2400), dict(top_k=1)]:
+        for u in (0.0, float(rng.random()), 1.0 - 2.0 ** -40):
+            tok, p = sample(_dev(l), u, context=_dev(ctx), **kw)
+            p = p.cpu().numpy().astype(np.float64)
+            ref, near = _sample64(l, ctx, **kw)
+            if near:
+                continue
+            assert np.array_equal(p > 0, ref > 0), (kw, (p > 0).sum(), (ref > 0).sum())
+            assert np.abs(p - ref).max() <= 2 ** -18 * ref.max(), kw
+            cdf = np.cumsum(p)
+            if u == 0.0:
+                assert tok == 0
+            elif u > cdf[-1]:
+                assert tok == n - 1
+            else:
+                assert p[tok] > 0 and cdf[tok] >= u - 1e-12 and cdf[tok] - p[tok] < u + 1e-12, (kw, u, tok)
+
+
+def test_sample_infinite_logit(gpu):
+    """+infinity at the top: its exponential is not a number, no probability is kept and the draw falls
+    back to the last token."""
+    from smallmind_amd.quantization import sample
+    l = np.random.default_rng(1).normal(0, 3, 32000).astype(np.float32)
+    l[77] = np.inf
+    for kw in (dict(top_k=40, top_p=0.9), dict(top_p=0.9)):
+        tok, p = sample(_dev(l), 0.5, **kw)
+        assert tok == 31999 and not bool((p != 0).any())
+
+
 def test_stream_read_runs_and_checks_its_size(gpu):
     """smx_stream_read (the bench's streaming-read ceiling) reads device memory without writing
     it, and refuses sizes that are not a positive multiple of 16 bytes."""
