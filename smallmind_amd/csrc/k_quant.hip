@@ -4,6 +4,8 @@
 // 419-917) element for element; Q8_0/Q4_0 encoders restate Q8Tensor.Quantize /
 // Q4Tensor.Quantize (Q8Tensor.cs:72-128, Q4Tensor.cs:75-134) at block 32 with an fp16 scale;
 // the K-quant encoders are this build's own and write the layout the reference decodes.
+#include <type_traits>
+
 #include "smx_formats.h"
 
 namespace smx {
@@ -14,308 +16,280 @@ constexpr int kThreads = 256;
 
 __device__ __forceinline__ float rd_half_exact(const uint8_t *p) { return h2f_exact(ld_u16(p)); }
 
-// ---- GGUF dequantization: one thread per 32 elements ---------------------------------------
-__device__ void unpack_k_scales(const uint8_t *s, uint32_t *sc, uint32_t *mn)
+// The codecs are bound by memory: 4 bytes per element on one side, and a block's bytes on the other.
+// A thread takes 4 elements, so that a wave reads or writes 1 KB of floats at once and the bytes of its
+// blocks (one K-quant block, eight of the 32-element ones) together; headers are read by all lanes of a
+// block from the same line, and an encoder's maxima are reduced over the lanes of its block.  Of 11.5 M
+// elements of Q4_K (53 MB each way, 10.6 us at the 5.0 TB/s of a large copy), one thread per block or
+// 32 elements, each with its own lines: encode 90 us, decode 125 us; now 28 and 21.
+
+// Bytes at any alignment (the hardware's unaligned access).
+template <typename T>
+__device__ __forceinline__ T ld_any(const uint8_t *p)
 {
-    sc[0] = s[0] & 0x3Fu;
-    sc[1] = (s[0] >> 6) | ((s[1] & 0x0Fu) << 2);
-    sc[2] = (s[1] >> 4) | ((s[2] & 0x03u) << 4);
-    sc[3] = (s[2] >> 2) & 0x3Fu;
-    sc[4] = s[3] & 0x3Fu;
-    sc[5] = (s[3] >> 6) | ((s[4] & 0x0Fu) << 2);
-    sc[6] = (s[4] >> 4) | ((s[5] & 0x03u) << 4);
-    sc[7] = (s[5] >> 2) & 0x3Fu;
-    mn[0] = s[6] & 0x3Fu;
-    mn[1] = (s[6] >> 6) | ((s[7] & 0x0Fu) << 2);
-    mn[2] = (s[7] >> 4) | ((s[8] & 0x03u) << 4);
-    mn[3] = (s[8] >> 2) & 0x3Fu;
-    mn[4] = s[9] & 0x3Fu;
-    mn[5] = (s[9] >> 6) | ((s[10] & 0x0Fu) << 2);
-    mn[6] = (s[10] >> 4) | ((s[11] & 0x03u) << 4);
-    mn[7] = (s[11] >> 2) & 0x3Fu;
+    T v;
+    __builtin_memcpy(&v, p, sizeof v);
+    return v;
+}
+template <typename T>
+__device__ __forceinline__ void st_any(uint8_t *p, T v) { __builtin_memcpy(p, &v, sizeof v); }
+
+template <int T>
+struct Type {
+    static constexpr bool k = T == SMX_TYPE_Q4_K || T == SMX_TYPE_Q5_K || T == SMX_TYPE_Q6_K;
+    static constexpr bool plain = T == SMX_TYPE_F32 || T == SMX_TYPE_F16;
+    static constexpr int elems = k ? 256 : plain ? 4 : 32;
+    static constexpr int bytes = T == SMX_TYPE_F32 ? 16 : T == SMX_TYPE_F16 ? 8 : T == SMX_TYPE_Q8_0 ? 34
+                               : T == SMX_TYPE_Q4_0 ? 18 : T == SMX_TYPE_Q4_K ? 144 : T == SMX_TYPE_Q5_K ? 176
+                               : T == SMX_TYPE_Q6_K ? 210 : T == SMX_TYPE_SMQ_Q8 ? 36 : 20;
+};
+
+// ---- GGUF dequantization --------------------------------------------------------------------
+__device__ __forceinline__ int nib(uint32_t n) { return n < 8u ? (int)n : (int)n - 16; }
+
+// 6-bit scale j of the packed scales at s (the minimums at s + 6)
+__device__ __forceinline__ uint32_t k_scale(const uint8_t *s, int j)
+{
+    const int k = (6 * j) >> 3, sh = (6 * j) & 7;
+    return (ld_any<uint16_t>(s + k) >> sh) & 63u;   // the byte after the last is masked away
 }
 
-__global__ void k_dequant_gguf(int type, const uint8_t *__restrict__ src, int64_t n,
-                               float *__restrict__ out)
+// Element v (of 256, 32 or 4) of block b.
+template <int T>
+__device__ __forceinline__ float decode_one(const uint8_t *b, int v)
 {
-    const int64_t chunk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t e0 = chunk * 32;
-    if (e0 >= n) return;
-    const int cnt = (int)(n - e0 < 32 ? n - e0 : 32);
-    float *y = out + e0;
-    if (type == SMX_TYPE_F32) {
-        const float *f = (const float *)src + e0;
-        for (int i = 0; i < cnt; i++) y[i] = f[i];
-    } else if (type == SMX_TYPE_F16) {
-        for (int i = 0; i < cnt; i++) y[i] = rd_half_exact(src + 2 * (e0 + i));
-    } else if (type == SMX_TYPE_SMQ_Q8 || type == SMX_TYPE_SMQ_Q4) {
+    if constexpr (T == SMX_TYPE_F32) {
+        return __uint_as_float(ld_any<uint32_t>(b + 4 * v));
+    } else if constexpr (T == SMX_TYPE_F16) {
+        return rd_half_exact(b + 2 * v);
+    } else if constexpr (T == SMX_TYPE_SMQ_Q8) {
         // Q8Tensor.Dequantize / Q4Tensor.Dequantize (Q8Tensor.cs:131-157, Q4Tensor.cs:150-178):
         // code * scale, one fp32 multiply; 32-element blocks of [fp32 scale | codes]
-        const bool q8 = type == SMX_TYPE_SMQ_Q8;
-        const uint8_t *b = src + chunk * (q8 ? 36 : 20);
-        const float d = __uint_as_float((uint32_t)b[0] | ((uint32_t)b[1] << 8) | ((uint32_t)b[2] << 16) |
-                                        ((uint32_t)b[3] << 24));
-        for (int i = 0; i < cnt; i++) {
-            int q;
-            if (q8) {
-                q = (int8_t)b[4 + i];
-            } else {
-                const uint32_t n = (b[4 + i / 2] >> (4 * (i & 1))) & 15u;
-                q = n < 8 ? (int)n : (int)n - 16;   // Q4Tensor.DecodeNibble (Q4Tensor.cs:140-143)
-            }
-            y[i] = (float)q * d;
-        }
-    } else if (type == SMX_TYPE_Q8_0) {   // GgufModelLoader.cs:464-492
-        const uint8_t *b = src + chunk * 34;
-        const float d = rd_half_exact(b);
-        for (int i = 0; i < cnt; i++) y[i] = (float)(int8_t)b[2 + i] * d;
-    } else if (type == SMX_TYPE_Q4_0) {   // GgufModelLoader.cs:494-534
-        const uint8_t *b = src + chunk * 18;
-        const float d = rd_half_exact(b);
-        for (int i = 0; i < cnt; i += 2) {
-            uint32_t packed = b[2 + i / 2];
-            int lo = (int)(packed & 15u), hi = (int)((packed >> 4) & 15u);
-            y[i] = (float)(lo < 8 ? lo : lo - 16) * d;
-            if (i + 1 < cnt) y[i + 1] = (float)(hi < 8 ? hi : hi - 16) * d;
-        }
+        return (float)(int8_t)b[4 + v] * __uint_as_float(ld_any<uint32_t>(b));
+    } else if constexpr (T == SMX_TYPE_SMQ_Q4) {   // Q4Tensor.DecodeNibble (Q4Tensor.cs:140-143)
+        return (float)nib((b[4 + v / 2] >> (4 * (v & 1))) & 15u) * __uint_as_float(ld_any<uint32_t>(b));
+    } else if constexpr (T == SMX_TYPE_Q8_0) {   // GgufModelLoader.cs:464-492
+        return (float)(int8_t)b[2 + v] * rd_half_exact(b);
+    } else if constexpr (T == SMX_TYPE_Q4_0) {   // GgufModelLoader.cs:494-534
+        return (float)nib((b[2 + v / 2] >> (4 * (v & 1))) & 15u) * rd_half_exact(b);
+    } else if constexpr (T == SMX_TYPE_Q6_K) {   // GgufModelLoader.cs:849-917, 16-element sub-blocks
+        const float sc = rd_half_exact(b + 208) * (float)(int8_t)b[192 + v / 16];
+        const uint32_t low4 = (b[v / 2] >> (4 * (v & 1))) & 15u;
+        const uint32_t high2 = (b[128 + v / 4] >> ((v % 4) * 2)) & 3u;
+        return sc * (float)((int)(low4 | (high2 << 4)) - 32);
     } else {
-        const int64_t sbi = e0 / 256;
-        const int j = (int)((e0 % 256) / 32);
-        if (type == SMX_TYPE_Q6_K) {   // GgufModelLoader.cs:849-917, 16-element sub-blocks
-            const uint8_t *b = src + sbi * 210;
-            const float d = rd_half_exact(b + 208);
-            for (int i = 0; i < cnt; i++) {
-                int v = j * 32 + i;
-                float sc = d * (float)(int8_t)b[192 + v / 16];
-                uint32_t low4 = (v % 2 == 0) ? (b[v / 2] & 15u) : ((b[v / 2] >> 4) & 15u);
-                uint32_t high2 = (b[128 + v / 4] >> ((v % 4) * 2)) & 3u;
-                int q = (int)(low4 | (high2 << 4));
-                y[i] = sc * (float)(q - 32);
-            }
-        } else {
-            const int bytes = type == SMX_TYPE_Q4_K ? 144 : 176;
-            const uint8_t *b = src + sbi * bytes;
-            const float d = rd_half_exact(b), dmin = rd_half_exact(b + 2);
-            uint32_t sc6[8], mn6[8];
-            unpack_k_scales(b + 4, sc6, mn6);
-            const float sc = d * (float)sc6[j];
-            const float m = dmin * (float)mn6[j];
-            if (type == SMX_TYPE_Q4_K) {   // GgufModelLoader.cs:657-741
-                // The reference loop runs i < count/2, so an odd tail element stays zero.
-                for (int i = 0; i < cnt; i++) y[i] = 0.0f;
-                for (int i = 0; i < cnt / 2; i++) {
-                    uint32_t packed = b[16 + j * 16 + i];
-                    float t0 = sc * (float)(packed & 15u);
-                    y[2 * i] = t0 - m;
-                    if (2 * i + 1 < cnt) {
-                        float t1 = sc * (float)((packed >> 4) & 15u);
-                        y[2 * i + 1] = t1 - m;
-                    }
-                }
-            } else {   // Q5_K, GgufModelLoader.cs:748-840
-                for (int i = 0; i < cnt; i++) {
-                    int v = j * 32 + i;
-                    uint32_t hb = ((b[16 + v / 8] >> (v % 8)) & 1u) << 4;
-                    uint32_t low4 = (v % 2 == 0) ? (b[48 + v / 2] & 15u) : ((b[48 + v / 2] >> 4) & 15u);
-                    int q = (int)(hb | low4) - 16;
-                    float t = sc * (float)q;
-                    y[i] = t - m;
-                }
-            }
+        const int j = v / 32;
+        const float sc = rd_half_exact(b) * (float)k_scale(b + 4, j);
+        const float m = rd_half_exact(b + 2) * (float)k_scale(b + 10, j);
+        if constexpr (T == SMX_TYPE_Q4_K) {   // GgufModelLoader.cs:657-741
+            const float t = sc * (float)((b[16 + v / 2] >> (4 * (v & 1))) & 15u);
+            return t - m;
+        } else {   // Q5_K, GgufModelLoader.cs:748-840
+            const uint32_t hb = ((b[16 + v / 8] >> (v % 8)) & 1u) << 4;
+            const uint32_t low4 = (b[48 + v / 2] >> (4 * (v & 1))) & 15u;
+            const float t = sc * (float)((int)(hb | low4) - 16);
+            return t - m;
         }
     }
 }
 
-// ---- encoders: one thread per block --------------------------------------------------------
+template <int T>
+__global__ void k_dequant_gguf(const uint8_t *__restrict__ src, int64_t n, float *__restrict__ out)
+{
+    const int64_t e0 = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    if (e0 >= n) return;
+    const uint8_t *b = src + e0 / Type<T>::elems * Type<T>::bytes;
+    const int v = (int)(e0 % Type<T>::elems);
+    if (e0 + 4 <= n && ((uintptr_t)out & 15) == 0) {
+        *(float4 *)(out + e0) = make_float4(decode_one<T>(b, v), decode_one<T>(b, v + 1), decode_one<T>(b, v + 2),
+                                            decode_one<T>(b, v + 3));
+        return;
+    }
+    for (int i = 0; i < 4 && e0 + i < n; i++) {
+        // the reference's Q4_K loop runs over whole pairs, so an odd last element stays zero
+        const bool half = T == SMX_TYPE_Q4_K && (i & 1) == 0 && e0 + i + 1 == n;
+        out[e0 + i] = half ? 0.0f : decode_one<T>(b, v + i);
+    }
+}
+
+// ---- encoders -------------------------------------------------------------------------------
 __device__ __forceinline__ float clampf(float v, float lo, float hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-__device__ float block_maxabs(const float *x, int n)
+// Maximum over groups of G lanes of values that are not NaN.
+template <int G>
+__device__ __forceinline__ float group_max(float m)
 {
-    float m = 0.0f;
-    for (int i = 0; i < n; i++) { float a = fabsf(x[i]); if (a > m) m = a; }
+#pragma unroll
+    for (int o = 1; o < G; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
     return m;
 }
 
-__device__ void st16(uint8_t *p, uint32_t h) { p[0] = (uint8_t)h; p[1] = (uint8_t)(h >> 8); }
-
-__device__ void pack_k_scales(const int *sc, const int *mn, uint8_t *s)
+// Largest magnitude of the group's elements, NaN left out
+template <int G>
+__device__ __forceinline__ float group_maxabs(const float *x)
 {
-    uint64_t a = 0, b = 0;
-    for (int j = 0; j < 8; j++) {
-        a |= (uint64_t)(sc[j] & 63) << (6 * j);
-        b |= (uint64_t)(mn[j] & 63) << (6 * j);
-    }
-    for (int i = 0; i < 6; i++) { s[i] = (uint8_t)(a >> (8 * i)); s[6 + i] = (uint8_t)(b >> (8 * i)); }
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) { const float a = fabsf(x[i]); if (a > m) m = a; }
+    return group_max<G>(m);
 }
 
-__device__ void enc_q8_0(const float *x, uint8_t *b)
+// the OR over the eight groups of 8 lanes of a wave
+__device__ __forceinline__ uint64_t or_groups(uint64_t v)
 {
-    float maxAbs = block_maxabs(x, 32);
-    float scale = maxAbs > 0.0f ? maxAbs / 127.0f : 1.0f;
-    float inv = 1.0f / scale;
-    st16(b, f2h_rne(scale));
-    for (int i = 0; i < 32; i++) {
-        float t = x[i] * inv;
-        b[2 + i] = (uint8_t)(int8_t)(int)rintf(clampf(t, -127.0f, 127.0f));
-    }
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1) v |= __shfl_xor((unsigned long long)v, o, 64);
+    return v;
 }
 
-__device__ void enc_q4_0(const float *x, uint8_t *b)
+// Q8_0 / Q4_0 and Q8Tensor.Quantize / Q4Tensor.Quantize (Q8Tensor.cs:72-128, Q4Tensor.cs:75-134) as
+// written, fp32 scale kept, at 32-element blocks (the SMQ upload layout: fp32 scale, then the codes).
+template <int T>
+__device__ __forceinline__ void encode32(const float *x, int v, uint8_t *b)
 {
-    float maxAbs = block_maxabs(x, 32);
-    float scale = maxAbs > 0.0f ? maxAbs / 7.0f : 1.0f;
-    float inv = 1.0f / scale;
-    st16(b, f2h_rne(scale));
-    for (int i = 0; i < 16; i++) {
-        float t0 = x[2 * i] * inv, t1 = x[2 * i + 1] * inv;
-        int c0 = (int)rintf(clampf(t0, -8.0f, 7.0f));
-        int c1 = (int)rintf(clampf(t1, -8.0f, 7.0f));
-        b[2 + i] = (uint8_t)((c0 & 0xF) | ((c1 & 0xF) << 4));
+    constexpr bool q8 = T == SMX_TYPE_Q8_0 || T == SMX_TYPE_SMQ_Q8, smq = T == SMX_TYPE_SMQ_Q8 || T == SMX_TYPE_SMQ_Q4;
+    constexpr int head = smq ? 4 : 2;
+    const float maxAbs = group_maxabs<8>(x);
+    const float scale = maxAbs > 0.0f ? maxAbs / (q8 ? 127.0f : 7.0f) : 1.0f;
+    const float inv = 1.0f / scale;
+    if (v == 0) {
+        if (smq) st_any<uint32_t>(b, __float_as_uint(scale));
+        else st_any<uint16_t>(b, (uint16_t)f2h_rne(scale));
     }
+    int c[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float t = x[i] * inv;
+        c[i] = (int)rintf(clampf(t, q8 ? -127.0f : -8.0f, q8 ? 127.0f : 7.0f));
+    }
+    if (q8)
+        st_any<uint32_t>(b + head + v, (uint32_t)(c[0] & 255) | (uint32_t)(c[1] & 255) << 8 |
+                                           (uint32_t)(c[2] & 255) << 16 | (uint32_t)(c[3] & 255) << 24);
+    else
+        st_any<uint16_t>(b + head + v / 2, (uint16_t)((c[0] & 15) | (c[1] & 15) << 4 | (c[2] & 15) << 8 | (c[3] & 15) << 12));
 }
 
-// Q8Tensor.Quantize / Q4Tensor.Quantize (Q8Tensor.cs:72-128, Q4Tensor.cs:75-134) as written, fp32
-// scale kept, at 32-element blocks: the SMQ upload layout (fp32 scale, then the codes).
-__device__ void enc_smq_q8(const float *x, uint8_t *b)
+// d, dmin and the packed scales of a K-quant block, by the lane of its first element
+__device__ __forceinline__ void put_k_header(uint8_t *b, int v, uint32_t d16, uint32_t m16, int ls, int lm)
 {
-    float maxAbs = block_maxabs(x, 32);
-    float scale = maxAbs > 0.0f ? maxAbs / 127.0f : 1.0f;
-    float inv = 1.0f / scale;
-    const uint32_t u = __float_as_uint(scale);
-    for (int i = 0; i < 4; i++) b[i] = (uint8_t)(u >> (8 * i));
-    for (int i = 0; i < 32; i++) {
-        float t = x[i] * inv;
-        b[4 + i] = (uint8_t)(int8_t)(int)rintf(clampf(t, -127.0f, 127.0f));
-    }
-}
-
-__device__ void enc_smq_q4(const float *x, uint8_t *b)
-{
-    float maxAbs = block_maxabs(x, 32);
-    float scale = maxAbs > 0.0f ? maxAbs / 7.0f : 1.0f;
-    float inv = 1.0f / scale;
-    const uint32_t u = __float_as_uint(scale);
-    for (int i = 0; i < 4; i++) b[i] = (uint8_t)(u >> (8 * i));
-    for (int i = 0; i < 16; i++) {
-        float t0 = x[2 * i] * inv, t1 = x[2 * i + 1] * inv;
-        int c0 = (int)rintf(clampf(t0, -8.0f, 7.0f));
-        int c1 = (int)rintf(clampf(t1, -8.0f, 7.0f));
-        b[4 + i] = (uint8_t)((c0 & 0xF) | ((c1 & 0xF) << 4));
+    const int j = v / 32;
+    const uint64_t s = or_groups((uint64_t)(ls & 63) << (6 * j)), m = or_groups((uint64_t)(lm & 63) << (6 * j));
+    if (v == 0) {
+        st_any<uint32_t>(b, d16 | m16 << 16);
+        st_any<uint32_t>(b + 4, (uint32_t)s);
+        st_any<uint32_t>(b + 8, (uint32_t)(s >> 32) | (uint32_t)m << 16);
+        st_any<uint32_t>(b + 12, (uint32_t)(m >> 16));
     }
 }
 
-__device__ void enc_q4_k(const float *x, uint8_t *b)
+__device__ __forceinline__ void encode_q4_k(const float *x, int v, uint8_t *b)
 {
-    float scl[8], mnv[8], maxs = 0.0f, maxm = 0.0f;
-    for (int j = 0; j < 8; j++) {
-        const float *s = x + 32 * j;
-        float lo = 0.0f, hi = s[0];
-        for (int i = 0; i < 32; i++) { if (s[i] < lo) lo = s[i]; if (s[i] > hi) hi = s[i]; }
-        scl[j] = (hi - lo) / 15.0f;
-        mnv[j] = -lo;
-        if (scl[j] > maxs) maxs = scl[j];
-        if (mnv[j] > maxm) maxm = mnv[j];
+    // lowest of the sub-block and 0, and highest, which is NaN if the first element is
+    float lo = 0.0f, hi = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; i++) { if (x[i] < lo) lo = x[i]; if (x[i] > hi) hi = x[i]; }
+    lo = -group_max<8>(-lo);
+    hi = group_max<8>(hi);
+    const float first = __shfl(x[0], (int)(threadIdx.x & 56), 64);
+    if (first != first) hi = first;
+    const float scl = (hi - lo) / 15.0f, mnv = -lo;
+    float maxs = 0.0f, maxm = 0.0f;
+    if (scl > maxs) maxs = scl;
+    if (mnv > maxm) maxm = mnv;
+    maxs = group_max<64>(maxs);
+    maxm = group_max<64>(maxm);
+    const uint32_t d16 = f2h_rne(maxs / 63.0f), m16 = f2h_rne(maxm / 63.0f);
+    const float df = h2f_exact(d16), mf = h2f_exact(m16);
+    const int ls = df > 0.0f ? (int)clampf(rintf(scl / df), 0.0f, 63.0f) : 0;
+    const int lm = mf > 0.0f ? (int)clampf(rintf(mnv / mf), 0.0f, 63.0f) : 0;
+    put_k_header(b, v, d16, m16, ls, lm);
+    const float sc = df * (float)ls, m = mf * (float)lm;
+    uint32_t q = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float t = x[i] + m;
+        q |= (uint32_t)(sc > 0.0f ? (int)clampf(rintf(t / sc), 0.0f, 15.0f) : 0) << (4 * i);
     }
-    uint32_t d16 = f2h_rne(maxs / 63.0f), m16 = f2h_rne(maxm / 63.0f);
-    float df = h2f_exact(d16), mf = h2f_exact(m16);
-    int ls[8], lm[8];
-    for (int j = 0; j < 8; j++) {
-        ls[j] = df > 0.0f ? (int)clampf(rintf(scl[j] / df), 0.0f, 63.0f) : 0;
-        lm[j] = mf > 0.0f ? (int)clampf(rintf(mnv[j] / mf), 0.0f, 63.0f) : 0;
+    st_any<uint16_t>(b + 16 + v / 2, (uint16_t)q);
+}
+
+__device__ __forceinline__ void encode_q5_k(const float *x, int v, uint8_t *b)
+{
+    const float scl = group_maxabs<8>(x) / 15.0f;
+    float maxs = 0.0f;
+    if (scl > maxs) maxs = scl;
+    maxs = group_max<64>(maxs);
+    const uint32_t d16 = f2h_rne(maxs / 63.0f);
+    const float df = h2f_exact(d16);
+    const int ls = df > 0.0f ? (int)clampf(rintf(scl / df), 0.0f, 63.0f) : 0;
+    put_k_header(b, v, d16, 0u, ls, 0);
+    const float sc = df * (float)ls;
+    uint32_t lo = 0, hi = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int q = sc > 0.0f ? (int)clampf(rintf(x[i] / sc), -16.0f, 15.0f) + 16 : 16;
+        lo |= (uint32_t)(q & 15) << (4 * i);
+        hi |= (uint32_t)(q >> 4 & 1) << i;
     }
-    st16(b, d16);
-    st16(b + 2, m16);
-    pack_k_scales(ls, lm, b + 4);
-    for (int j = 0; j < 8; j++) {
-        float sc = df * (float)ls[j];
-        float m = mf * (float)lm[j];
-        for (int i = 0; i < 16; i++) {
-            int q[2];
-            for (int t = 0; t < 2; t++) {
-                float v = x[32 * j + 2 * i + t] + m;
-                q[t] = sc > 0.0f ? (int)clampf(rintf(v / sc), 0.0f, 15.0f) : 0;
-            }
-            b[16 + 16 * j + i] = (uint8_t)(q[0] | (q[1] << 4));
+    st_any<uint16_t>(b + 48 + v / 2, (uint16_t)lo);
+    hi |= __shfl_xor(hi, 1, 64) << 4;
+    if ((v & 4) == 0) b[16 + v / 8] = (uint8_t)hi;
+}
+
+__device__ __forceinline__ void encode_q6_k(const float *x, int v, uint8_t *b)
+{
+    const float scl = group_maxabs<4>(x) / 31.0f;
+    float maxs = 0.0f;
+    if (scl > maxs) maxs = scl;
+    maxs = group_max<64>(maxs);
+    const uint32_t d16 = f2h_rne(maxs / 127.0f);
+    const float df = h2f_exact(d16);
+    const int ls = df > 0.0f ? (int)clampf(rintf(scl / df), -128.0f, 127.0f) : 0;
+    const float sc = df * (float)ls;
+    uint32_t lo = 0, hi = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int q = sc > 0.0f ? (int)clampf(rintf(x[i] / sc), -32.0f, 31.0f) + 32 : 32;
+        lo |= (uint32_t)(q & 15) << (4 * i);
+        hi |= (uint32_t)(q >> 4 & 3) << (2 * i);
+    }
+    st_any<uint16_t>(b + v / 2, (uint16_t)lo);
+    b[128 + v / 4] = (uint8_t)hi;
+    if ((v & 15) == 0) b[192 + v / 16] = (uint8_t)(int8_t)ls;
+    if (v == 0) st_any<uint16_t>(b + 208, (uint16_t)d16);
+}
+
+// n is a multiple of the block size; F16 has blocks of one element.
+template <int T>
+__global__ void k_quantize(const float *__restrict__ x, int64_t n, uint8_t *__restrict__ out)
+{
+    const int64_t e0 = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    if (e0 >= n) return;   // whole groups of lanes: blocks are multiples of 32 elements
+    uint8_t *b = out + e0 / Type<T>::elems * Type<T>::bytes;
+    const int v = (int)(e0 % Type<T>::elems);
+    float f[4];
+    if (e0 + 4 <= n && ((uintptr_t)x & 15) == 0) {
+        const float4 q = *(const float4 *)(x + e0);
+        f[0] = q.x, f[1] = q.y, f[2] = q.z, f[3] = q.w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) f[i] = e0 + i < n ? x[e0 + i] : 0.0f;
+    }
+    if constexpr (T == SMX_TYPE_Q4_K) {
+        encode_q4_k(f, v, b);
+    } else if constexpr (T == SMX_TYPE_Q5_K) {
+        encode_q5_k(f, v, b);
+    } else if constexpr (T == SMX_TYPE_Q6_K) {
+        encode_q6_k(f, v, b);
+    } else if constexpr (T == SMX_TYPE_F16) {
+        if (e0 + 4 <= n) {
+            st_any<uint64_t>(b, (uint64_t)(f2h_rne(f[0]) | f2h_rne(f[1]) << 16) |
+                                    (uint64_t)(f2h_rne(f[2]) | f2h_rne(f[3]) << 16) << 32);
+        } else {
+            for (int i = 0; e0 + i < n; i++) st_any<uint16_t>(b + 2 * i, (uint16_t)f2h_rne(f[i]));
         }
-    }
-}
-
-__device__ void enc_q5_k(const float *x, uint8_t *b)
-{
-    float scl[8], maxs = 0.0f;
-    for (int j = 0; j < 8; j++) {
-        scl[j] = block_maxabs(x + 32 * j, 32) / 15.0f;
-        if (scl[j] > maxs) maxs = scl[j];
-    }
-    uint32_t d16 = f2h_rne(maxs / 63.0f);
-    float df = h2f_exact(d16);
-    int ls[8], lm[8];
-    for (int j = 0; j < 8; j++) {
-        ls[j] = df > 0.0f ? (int)clampf(rintf(scl[j] / df), 0.0f, 63.0f) : 0;
-        lm[j] = 0;
-    }
-    for (int i = 0; i < 176; i++) b[i] = 0;
-    st16(b, d16);
-    pack_k_scales(ls, lm, b + 4);
-    uint8_t *qh = b + 16, *ql = b + 48;
-    for (int j = 0; j < 8; j++) {
-        float sc = df * (float)ls[j];
-        for (int i = 0; i < 32; i++) {
-            int v = 32 * j + i;
-            int q = sc > 0.0f ? (int)clampf(rintf(x[v] / sc), -16.0f, 15.0f) + 16 : 16;
-            if (q & 16) qh[v / 8] |= (uint8_t)(1u << (v % 8));
-            if (v % 2 == 0) ql[v / 2] |= (uint8_t)(q & 0xF);
-            else ql[v / 2] |= (uint8_t)((q & 0xF) << 4);
-        }
-    }
-}
-
-__device__ void enc_q6_k(const float *x, uint8_t *b)
-{
-    float scl[16], maxs = 0.0f;
-    for (int j = 0; j < 16; j++) {
-        scl[j] = block_maxabs(x + 16 * j, 16) / 31.0f;
-        if (scl[j] > maxs) maxs = scl[j];
-    }
-    uint32_t d16 = f2h_rne(maxs / 127.0f);
-    float df = h2f_exact(d16);
-    for (int i = 0; i < 210; i++) b[i] = 0;
-    uint8_t *ql = b, *qh = b + 128;
-    for (int j = 0; j < 16; j++) {
-        int ls = df > 0.0f ? (int)clampf(rintf(scl[j] / df), -128.0f, 127.0f) : 0;
-        b[192 + j] = (uint8_t)(int8_t)ls;
-        float sc = df * (float)ls;
-        for (int i = 0; i < 16; i++) {
-            int v = 16 * j + i;
-            int q = sc > 0.0f ? (int)clampf(rintf(x[v] / sc), -32.0f, 31.0f) + 32 : 32;
-            if (v % 2 == 0) ql[v / 2] |= (uint8_t)(q & 0xF);
-            else ql[v / 2] |= (uint8_t)((q & 0xF) << 4);
-            qh[v / 4] |= (uint8_t)(((q >> 4) & 3) << ((v % 4) * 2));
-        }
-    }
-    st16(b + 208, d16);
-}
-
-__global__ void k_quantize(int type, const float *__restrict__ x, int64_t nblocks,
-                           uint8_t *__restrict__ out)
-{
-    const int64_t blk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (blk >= nblocks) return;
-    switch (type) {
-    case SMX_TYPE_Q8_0: enc_q8_0(x + blk * 32, out + blk * 34); break;
-    case SMX_TYPE_Q4_0: enc_q4_0(x + blk * 32, out + blk * 18); break;
-    case SMX_TYPE_Q4_K: enc_q4_k(x + blk * 256, out + blk * 144); break;
-    case SMX_TYPE_Q5_K: enc_q5_k(x + blk * 256, out + blk * 176); break;
-    case SMX_TYPE_Q6_K: enc_q6_k(x + blk * 256, out + blk * 210); break;
-    case SMX_TYPE_SMQ_Q8: enc_smq_q8(x + blk * 32, out + blk * 36); break;
-    case SMX_TYPE_SMQ_Q4: enc_smq_q4(x + blk * 32, out + blk * 20); break;
-    case SMX_TYPE_F16: {
-        uint32_t h = f2h_rne(x[blk]);
-        out[2 * blk] = (uint8_t)h;
-        out[2 * blk + 1] = (uint8_t)(h >> 8);
-        break;
-    }
-    default: break;
+    } else {
+        encode32<T>(f, v, b);
     }
 }
 
@@ -413,6 +387,24 @@ __global__ void k_dequant_smx(WView w, int64_t row0, int64_t nrows, float *__res
 
 unsigned grid_for(int64_t n) { return (unsigned)((n + kThreads - 1) / kThreads); }
 
+template <typename F>
+hipError_t by_type(int type, F f)
+{
+    switch (type) {
+    case SMX_TYPE_F32: f(std::integral_constant<int, SMX_TYPE_F32>{}); break;
+    case SMX_TYPE_F16: f(std::integral_constant<int, SMX_TYPE_F16>{}); break;
+    case SMX_TYPE_Q4_0: f(std::integral_constant<int, SMX_TYPE_Q4_0>{}); break;
+    case SMX_TYPE_Q8_0: f(std::integral_constant<int, SMX_TYPE_Q8_0>{}); break;
+    case SMX_TYPE_Q4_K: f(std::integral_constant<int, SMX_TYPE_Q4_K>{}); break;
+    case SMX_TYPE_Q5_K: f(std::integral_constant<int, SMX_TYPE_Q5_K>{}); break;
+    case SMX_TYPE_Q6_K: f(std::integral_constant<int, SMX_TYPE_Q6_K>{}); break;
+    case SMX_TYPE_SMQ_Q8: f(std::integral_constant<int, SMX_TYPE_SMQ_Q8>{}); break;
+    case SMX_TYPE_SMQ_Q4: f(std::integral_constant<int, SMX_TYPE_SMQ_Q4>{}); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 }  // namespace
 
 int fmt_from_type(int type)
@@ -433,23 +425,22 @@ int fmt_from_type(int type)
 
 hipError_t launch_dequant_gguf(int type, const void *blocks, int64_t n, float *out, hipStream_t s)
 {
-    const int64_t chunks = (n + 31) / 32;
-    if (chunks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_dequant_gguf, dim3(grid_for(chunks)), dim3(kThreads), 0, s, type,
-                       (const uint8_t *)blocks, n, out);
-    return hipGetLastError();
+    if (n == 0) return hipSuccess;
+    const dim3 grid(grid_for((n + 3) / 4));
+    return by_type(type, [&](auto t) {
+        hipLaunchKernelGGL((k_dequant_gguf<decltype(t)::value>), grid, dim3(kThreads), 0, s, (const uint8_t *)blocks, n,
+                           out);
+    });
 }
 
 hipError_t launch_quantize_gguf(int type, const float *x, int64_t n, void *blocks, hipStream_t s)
 {
-    const int be = type == SMX_TYPE_F16 ? 1
-                 : (type == SMX_TYPE_Q8_0 || type == SMX_TYPE_Q4_0 || type == SMX_TYPE_SMQ_Q8 || type == SMX_TYPE_SMQ_Q4)
-                     ? 32 : 256;
-    const int64_t nblocks = n / be;
-    if (nblocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_quantize, dim3(grid_for(nblocks)), dim3(kThreads), 0, s, type, x, nblocks,
-                       (uint8_t *)blocks);
-    return hipGetLastError();
+    if (n == 0) return hipSuccess;
+    const dim3 grid(grid_for((n + 3) / 4));
+    return by_type(type, [&](auto t) {
+        if constexpr (decltype(t)::value != SMX_TYPE_F32)
+            hipLaunchKernelGGL((k_quantize<decltype(t)::value>), grid, dim3(kThreads), 0, s, x, n, (uint8_t *)blocks);
+    });
 }
 
 hipError_t launch_fill_normal(uint64_t seed, int64_t n, float std, float *out, hipStream_t s)

@@ -70,6 +70,37 @@ def test_device_encoder_matches_oracle_bytes(gpu, name):
     assert np.array_equal(got, O.quantize(qt, x))
 
 
+@pytest.mark.parametrize("name", list(ALL_TYPES))
+@pytest.mark.parametrize("nblocks", [1, 3, 65])
+def test_codecs_at_any_alignment(gpu, name, nblocks):
+    """Four elements per thread: results and bytes are those of the oracle for blocks at an odd address
+    (encoded through the C entry point too), floats at one that is only a multiple of 4, and every
+    length of the last group; encoders keep what lies beside their output."""
+    import torch
+
+    from smallmind_amd._lib import call
+    from smallmind_amd.quantization import dequantize
+    qt = ALL_TYPES[name]
+    be, s = O.BLOCK_ELEMS[qt], torch.cuda.current_stream().cuda_stream
+    b = random_blocks(qt, nblocks, nblocks)
+    odd = _dev(b) if name == "F32" else _dev(np.concatenate([np.zeros(1, np.uint8), b]))[1:]
+    out = torch.full((nblocks * be + 5,), 7.0, device="cuda")
+    for n in {max(1, nblocks * be - k) for k in range(6)}:
+        ref = O.dequant(qt, b, n)
+        assert np.array_equal(dequantize(qt, odd, n).cpu().numpy().view(np.uint32), ref.view(np.uint32))
+        out.fill_(7.0)
+        call("smx_dequant", int(qt), odd.data_ptr(), n, out.data_ptr() + 4, s)
+        assert np.array_equal(out.cpu().numpy()[1:1 + n].view(np.uint32), ref.view(np.uint32))
+        assert bool((out[1 + n:] == 7.0).all()) and float(out[0]) == 7.0
+    if name == "F32":
+        return
+    x = np.random.default_rng(nblocks).normal(0, 1, nblocks * be + 1).astype(np.float32)
+    got, xd = torch.full((b.size + 2,), 0xA5, dtype=torch.uint8, device="cuda"), _dev(x)
+    call("smx_quantize", int(qt), xd.data_ptr() + 4, nblocks * be, got.data_ptr() + 1, s)
+    got = got.cpu().numpy()
+    assert np.array_equal(got[1:-1], O.quantize(qt, x[1:])) and got[0] == got[-1] == 0xA5
+
+
 def test_fill_normal_statistics(gpu):
     from smallmind_amd.quantization import fill_normal
     v = fill_normal(5, 1_000_001, 0.02).cpu().numpy().astype(np.float64)
