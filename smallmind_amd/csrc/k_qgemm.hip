@@ -1091,20 +1091,24 @@ __global__ __launch_bounds__(256) void k_qprep_long(const float *__restrict__ x,
     }
 }
 
-// More than 16 tokens: a workgroup takes 4 tokens (a quarter of a token tile), thread (item lane
+// More than 16 tokens, or no norm: a workgroup takes 4 tokens (a quarter of a token tile), thread (item lane
 // tid / 4, token tid % 4).  Four neighbouring lanes store the same item of four tokens, 64
 // contiguous bytes of a part (one token per workgroup stored 16-byte pieces 256 bytes apart, which
 // ran at a third of the copy rate).  The rows of a norm are read again from the L1 for the
 // second pass instead of being held in registers.  SUMS: the kind of sub-block sums written (xp_sums).
+// Without a norm no thread needs the whole row, and the rows are cut into spans of items as well
+// (qprep_span): what bounds few tokens is the chain of loads in the few workgroups that four tokens
+// each make.
 template <int PRO, int SUMS>
 __global__ __launch_bounds__(256) void k_qprep_tokens(const float *__restrict__ x, int64_t x_stride, int M, int K,
                                                       const float *__restrict__ gamma,
                                                       const float *__restrict__ beta, float eps,
-                                                      uint8_t *__restrict__ xp)
+                                                      uint8_t *__restrict__ xp, int span)
 {
     __shared__ float red[4][4];
     const int nsb = K >> 5, items = K >> 3, ntt = (M + 15) >> 4;
     const int tid = threadIdx.x, tq = tid & 3, i0 = tid >> 2;
+    const int first = (int)blockIdx.y * span, end = min(items, first + span);   // this workgroup's items
     const int m = blockIdx.x * 4 + tq, tt = m >> 4, t = m & 15;
     const bool live = m < M;
     const float4 *xr = (const float4 *)(x + (int64_t)min(m, M - 1) * x_stride);
@@ -1143,7 +1147,7 @@ __global__ __launch_bounds__(256) void k_qprep_tokens(const float *__restrict__ 
     }
     uint8_t *xt = xp + (size_t)tt * nsb * 3072u + t * 16;
 #pragma unroll 2
-    for (int i = i0; i < items; i += 64) {
+    for (int i = first + i0; i < end; i += 64) {
         float v[8];
         unpack8(xr[2 * i], xr[2 * i + 1], v);
         if constexpr (PRO != PRO_NONE) {
@@ -1181,6 +1185,17 @@ __global__ __launch_bounds__(256) void k_qprep_tokens(const float *__restrict__ 
             *(uint4 *)(p + 1024 * pt) = make_uint4(w[0], w[1], w[2], w[3]);
         }
     }
+}
+
+// Items per workgroup of k_qprep_tokens: the whole row under a norm (its statistic); else one item
+// per thread, and more only where that would make over 2048 workgroups (eight per CU).  Per call of the
+// operator: 16 tokens of 8192 18.3 us (16 workgroups of whole rows in k_qprep, 5.1 us of it) -> 17.6; from
+// 511 tokens on, whole rows and spans are within 1 % of each other.
+unsigned qprep_span(unsigned groups, unsigned items, int pro)
+{
+    if (pro != PRO_NONE) return items;
+    const unsigned steps = (items + 63) / 64;   // 64 items at a time
+    return 64 * std::max(1u, (groups * steps + 2047) / 2048);
 }
 
 template <int F, int RT, int TT, int NW, int SB>
@@ -1354,9 +1369,10 @@ hipError_t launch_qgemm(const QgemmArgs &a, const float *x, int64_t x_stride, in
     const unsigned mp = (unsigned)((a.M + 15) / 16 * 16);
     int ipt = (K / 8 + 255) / 256;
 #define SMX_QPREP(KN) hipLaunchKernelGGL(KN, dim3(mp), dim3(256), 0, s, x, x_stride, a.M, K, pro, gamma, beta, eps, (uint8_t *)a.xp)
-#define SMX_QPREPT(P, S) hipLaunchKernelGGL((k_qprep_tokens<P, S>), dim3(mp / 4), dim3(256), 0, s, x, x_stride, a.M, K, gamma, beta, eps, (uint8_t *)a.xp)
+    const unsigned span = qprep_span(mp / 4, K / 8, pro);
+#define SMX_QPREPT(P, S) hipLaunchKernelGGL((k_qprep_tokens<P, S>), dim3(mp / 4, (K / 8 + span - 1) / span), dim3(256), 0, s, x, x_stride, a.M, K, gamma, beta, eps, (uint8_t *)a.xp, (int)span)
     if (!x) ipt = -1;   // the parts are already in a.xp (written by the producing kernel)
-    if (x && a.M > 16) {
+    if (x && (a.M > 16 || pro == PRO_NONE)) {
         const int kind = qgemm_sums_kind(a.w, a.M);
 #define SMX_QPREPP(P) do { if (kind == 0) SMX_QPREPT(P, 0); else if (kind == 1) SMX_QPREPT(P, 1); else SMX_QPREPT(P, 2); } while (0)
         if (pro == PRO_NONE) SMX_QPREPP(PRO_NONE);

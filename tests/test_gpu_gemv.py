@@ -171,6 +171,25 @@ def test_matmul_tile_kernel_vs_float64(gpu, name, m, N, K):
     assert worst <= 1.0, worst
 
 
+@pytest.mark.parametrize("name,m,K", [("Q8_0", 5, 544),     # one span of 64 eight-element items and one of 4
+                                      ("Q4_0", 16, 4128),   # nine spans, the last of 4 items
+                                      ("Q5_K", 13, 8448),   # padding tokens in the last group of four
+                                      ("Q4_K", 2500, 2304),  # spans of 128 items with sub-block sums, the last of 32
+                                      ("Q6_K", 2500, 2304)])  # the same with sums of half sub-blocks
+def test_matmul_activation_spans_vs_float64(gpu, name, m, K):
+    """Activation parts written by several workgroups per row, at ragged last spans; the GEMM bound
+    of this file per output."""
+    qt, N = TYPES[name], 40
+    W = quantized(qt, (N, K), seed=m + K)
+    X = np.random.default_rng(m + K).normal(0, 1, (m, K)).astype(np.float32)
+    Y = _dev(_gemv(qt, W, N, K, X, m=m)).double()
+    Wf = _dev(O.dequant(qt, W, N * K).reshape(N, K)).double()
+    Xd = _dev(X).double()
+    ref, scale = Xd @ Wf.t(), Xd.abs() @ Wf.abs().t()
+    worst = float(((Y - ref).abs() / (TIGHT * scale + 1e-30)).max())
+    assert worst <= 1.0, worst
+
+
 def test_fused_equals_dequant_then_matmul(gpu):
     """The reference's live equivalence check (ExpandedQuantizationTests.cs:229-250): fused
     quantized matmul == dequantize then fp32 matmul."""
