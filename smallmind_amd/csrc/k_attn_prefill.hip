@@ -105,6 +105,32 @@ __device__ __forceinline__ void split8(const float *v, uint4 *o)
     }
 }
 
+// Beyond this an element has no finite bf16 part (infinities among them), and its part products would be
+// NaN where fp32 arithmetic has a value.
+constexpr float kPartMax = 3.38e38f;
+
+// One query of kHD dimensions (scaled) against keys 0 .. n - 1 by one wave, in fp32: the output of
+// dimension `lane`.
+__device__ __noinline__ float attend_fp32(const float *qr, float scale, const float *K, const float *V, int ctx_stride, int n)
+{
+    const int lane = threadIdx.x & 63;
+    auto score = [&](int j) {
+        float s = 0.0f;
+        for (int e = 0; e < kHD; e++) s = __builtin_fmaf(qr[e] * scale, K[(int64_t)e * ctx_stride + j], s);
+        return s;
+    };
+    float mx = -INFINITY, sum = 0.0f, acc = 0.0f;
+    for (int j = lane; j < n; j += 64) mx = fmaxf(mx, score(j));
+    for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    for (int j0 = 0; j0 < n; j0 += 64) {
+        const float w = j0 + lane < n ? fastexp(score(j0 + lane) - mx) : 0.0f;
+        sum += w;
+        for (int i = 0; i < min(64, n - j0); i++) acc = __builtin_fmaf(__shfl(w, i, 64), V[(int64_t)(j0 + i) * kHD + lane], acc);
+    }
+    for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
+    return acc * (1.0f / sum);
+}
+
 // With pb.blk set (several sessions' runs of a batch in one launch), a workgroup's rows, cache
 // and first position come from the block table instead of the arguments: q, out and tok_off
 // move to the block's first batch row, and the block is a run of M <= TT tokens at t0 = 0.
@@ -125,6 +151,13 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
         float o[KW > 1 ? KW - 1 : 1][RW][2 * 16][64];
     };
     __shared__ __align__(16) uint8_t s_mem[sizeof(Lds)];
+    __shared__ int s_large;   // an operand beyond kPartMax
+    float large = 0.0f;
+    auto note8 = [&](const float *x) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) large = fmaxf(large, fabsf(x[e]));
+    };
+    if (threadIdx.x == 0) s_large = 0;   // (read after the loops' barriers)
     static_assert(KW == 1 || sizeof(Red) <= sizeof(uint4) * KW * 2 * 4 * 3 * 2 * kKeys * 2, "outputs reuse the tiles");
     Lds &L = *(Lds *)s_mem;
     Red &R = *(Red *)s_mem;
@@ -160,6 +193,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
 #pragma unroll
             for (int e = 0; e < 8; e++) x[e] = qr[16 * t + 8 * h + e] * scale;   // (scalar loads: q is 4-byte aligned)
             uint4 p[3];
+            note8(x);
             split8(x, p);
 #pragma unroll
             for (int c = 0; c < 3; c++) L.q[rw][t][c][lane] = p[c];
@@ -198,6 +232,14 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
             for (int c = 0; c < 3; c++) L.k[kg][slot][dg >> 1][c][dg & 1][i & 31] = p[c];
         }
     };
+    auto note_k = [&](int tile) {   // (keys past the written ones may hold anything)
+#pragma unroll
+        for (int n = 0; n < IT; n++) {
+            const float was = large;
+            note8(kr[n]);
+            large = kKeys * tile + ((tg + 64 * RW * n) & 31) < n_max ? large : was;
+        }
+    };
     auto load_v = [&](int tile) {
         const int t = min(tile, (ctx_stride - 1) / kKeys);
         const char *b = Vb + 4u * (uint32_t)(kKeys * t * kHD);
@@ -229,6 +271,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
                 vr[n][e] = key < n_max ? vr[n][e] : 0.0f;
             }
             uint4 p[3];
+            note8(vr[n]);
             split8(vr[n], p);
 #pragma unroll
             for (int c = 0; c < 3; c++) L.v[kg][slot][c][sh >> 1][sh & 1][i & 63] = p[c];
@@ -263,6 +306,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
     // (the next tile is split under the current one's products, the one after it is in flight)
     float mx = -INFINITY;
     load_k(kg);
+    note_k(kg);
     store_k(0);
     load_k(kg + KW);
     __syncthreads();
@@ -270,6 +314,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
         const int tile = kg + KW * it;
         f32x16 s;
         scores(it & 1, s);
+        note_k(tile + KW);
         store_k((it + 1) & 1);
         load_k(tile + 2 * KW);
 #pragma unroll
@@ -367,6 +412,28 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
     for (; it < n_it; it += 2) {
         pass2(it, s0, s1, std::true_type{}, std::true_type{});
         if (it + 1 < n_it) pass2(it + 1, s1, s0, std::true_type{}, std::true_type{});
+    }
+    if (large > kPartMax) s_large = 1;
+    __syncthreads();
+    if (s_large) {   // uniform: the workgroup's rows again in fp32, a row per wave at a time
+        for (int r = wv; r < 32 * RW; r += RW * KW) {
+            const int t = t0 + r / G, hd = kvh * G + r % G;
+            if (t >= M) break;
+            const float o = attend_fp32(q + (int64_t)t * q_stride + (int64_t)hd * kHD, scale, K, V, ctx_stride, p_first + t + 1);
+            if (!out_parts) {
+                out[(int64_t)t * out_stride + (int64_t)hd * kHD + lane] = o;
+                continue;
+            }
+            const int nsb = n_head * kHD / 32;
+            xp_store(out_parts, nsb, tok_off + t, hd * kHD + lane, o);
+            if (sums.kind) {
+                float a = o;   // sum over 16 dimensions
+                for (int x = 1; x < 16; x <<= 1) a += __shfl_xor(a, x, 64);
+                const float b = __shfl_xor(a, 16, 64);
+                if ((lane & 31) == 0) xp_sums(out_parts, sums.kind, sums.M, nsb, tok_off + t, hd * (kHD / 32) + lane / 32, a, b);
+            }
+        }
+        return;
     }
     sum += half_other(sum);
     if constexpr (KW > 1) {   // the key groups' sums and outputs, added in order by group 0

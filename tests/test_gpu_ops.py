@@ -228,6 +228,32 @@ def test_sample_vs_oracle(gpu, n, opts):
             assert tok == otok, (u, tok, otok)
 
 
+def test_attention_prefill_many_rows_infinities(gpu):
+    """Infinite and nearly overflowing cache entries, which have no finite bf16 parts, give what the
+    fp32 kernel of short runs gives for the same tokens (the op bound of this file)."""
+    import torch
+    from smallmind_amd.quantization import attention_prefill
+    H, Hkv, hd, n, ctx = 32, 4, 64, 416, 420
+    g = torch.Generator("cuda").manual_seed(5)
+    q = torch.randn(n, H, hd, device="cuda", generator=g)
+    k = torch.randn(Hkv, hd, ctx, device="cuda", generator=g)
+    v = torch.randn(Hkv, ctx, hd, device="cuda", generator=g)
+    v[0, 5, 3] = float("inf")
+    v[1, 40, 7] = 3.4e38
+    k[2, 11, 9] = float("inf")
+    k[:, :, n:] = float("inf")    # not written: read by no token
+    v[:, n:] = float("inf")
+    got = attention_prefill(q, k, v, H, Hkv, hd, ctx, 0, n).reshape(n, H, hd)
+    few = attention_prefill(q[n - 16:].contiguous(), k, v, H, Hkv, hd, ctx, n - 16, 16).reshape(16, H, hd)
+    got = got[n - 16:]
+    assert torch.isinf(few[:, :8, 3]).all() and torch.isfinite(few[:, 24:]).all()
+    fin = torch.isfinite(few)
+    assert torch.equal(fin, torch.isfinite(got)) and torch.equal(got.isnan(), few.isnan())
+    assert torch.equal(got[few.isinf()], few[few.isinf()])
+    err = (got - few).abs().double() / few.abs().double().clamp(min=1.0)
+    assert float(err[fin].max()) < 2e-5
+
+
 def _sample64(l, ctx, temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, repetition_penalty=1.0, frequency_penalty=0.0,
               repetition_window=0):
     """Float32 logits stages, float64 probabilities: (probabilities, whether a cutoff lies within rounding)."""
