@@ -3,7 +3,7 @@
 // GGUF-layout dequantization restates GgufModelLoader.Convert*Tensor (GgufModelLoader.cs:
 // 419-917) element for element; Q8_0/Q4_0 encoders restate Q8Tensor.Quantize /
 // Q4Tensor.Quantize (Q8Tensor.cs:72-128, Q4Tensor.cs:75-134) at block 32 with an fp16 scale;
-// the K-quant encoders are this build's own and write the layout the reference decodes.
+// the K-quant encoders (the reference has none) write the layout that the reference decodes.
 #include <type_traits>
 
 #include "smx_formats.h"
