@@ -189,7 +189,8 @@ typedef struct smx_sampling {
  * :628-936 and SampleFromProbs :708-724).  logits (n floats) and context (n_context token ids,
  * oldest first) are device memory; u in [0, 1) is the uniform draw the reference takes from
  * Random.NextDouble.  probs (n floats, device) receives the final distribution and token
- * (device) the sampled id.  Ties at the top-k / top-p cutoffs are all kept. */
+ * (device) the sampled id; probs may be the logits' own buffer.  Ties at the top-k / top-p cutoffs
+ * are all kept. */
 SMX_API int smx_sample(const float *logits_dev, int n, const int32_t *context_dev, int n_context,
                        const smx_sampling *params, double u, float *probs_dev, int32_t *token_dev,
                        void *stream);

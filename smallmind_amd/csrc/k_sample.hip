@@ -184,6 +184,7 @@ __device__ __forceinline__ T wave_scan(T v, int lane)   // inclusive
 
 // Penalties: each distinct token of the window w once, by the first thread that holds it.  The new
 // value, times scale, goes to where the old one is held; for one in registers it goes to mem[t], marked by a bit.
+// (logits[t] is read before anything is stored for token t, so mem may be the logits' own buffer.)
 template <int R>
 __device__ __forceinline__ void penalise(SampleShared &S, Vals<R> &x, const float *__restrict__ logits,
                                          const int32_t *w, int nw, const smx_sampling &sp, float scale)
@@ -462,12 +463,15 @@ __device__ __forceinline__ int sample_pipeline(const float *__restrict__ logits,
     x.lds = values;
     x.mem = probs;
     x.n = n;
-    // 2. temperature, applied to each value as it is first held (x 1 is exact)
-    const float scale = sp.temperature != 1.0f ? 1.0f / sp.temperature : 1.0f;
+    // 2. temperature, applied to each value as it is first held (x 1 is exact).  Where the values are held in
+    // the logits' own buffer (probs == logits), the penalties still need the unscaled ones: scaled after them
+    const bool penalties = sp.repetition_penalty != 1.0f || sp.presence_penalty != 0.0f || sp.frequency_penalty != 0.0f;
+    const bool late = R < 0 && penalties && logits == probs;
+    const float temp = sp.temperature != 1.0f ? 1.0f / sp.temperature : 1.0f, scale = late ? 1.0f : temp;
     x.load(logits, scale);
 
     // 1. penalties
-    if (sp.repetition_penalty != 1.0f || sp.presence_penalty != 0.0f || sp.frequency_penalty != 0.0f) {
+    if (penalties) {
         const int win = sp.repetition_window > 0 ? sp.repetition_window : min(n_ctx, 256);
         const int start = max(0, n_ctx - win), nw = n_ctx - start;
         if (R > 0) S.bits[tid] = 0;
@@ -482,6 +486,7 @@ __device__ __forceinline__ int sample_pipeline(const float *__restrict__ logits,
             x.rows([&](int row, float &f) {
                 if ((S.bits[((row - kRows * kT) >> 5) + (tid >> 5)] >> (tid & 31)) & 1u) f = (probs + row)[tid];
             }, std::make_integer_sequence<int, R>{});
+        if (late) x.each([&](int, float l) { return l * temp; });
     }
     BlockSum sum(S);
     // 3. top-k

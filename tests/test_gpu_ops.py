@@ -330,6 +330,32 @@ def test_sample_infinite_logit(gpu):
         assert tok == 31999 and not bool((p != 0).any())
 
 
+@pytest.mark.parametrize("n", [1000, 40000, 65536, 65537, 90001])
+def test_sample_in_place(gpu, n):
+    """probs may be the logits' own buffer: the same token and the same bits as in one of its own, with
+    the values on the compute unit and, above 65536, in that buffer."""
+    import ctypes
+
+    import torch
+
+    from smallmind_amd._lib import SamplingC, call
+    rng = np.random.default_rng(n)
+    l = _dev(rng.normal(0, 3, n).astype(np.float32))
+    ctx = _dev(rng.integers(0, n, 300).astype(np.int32))
+    for temp, top_k, top_p, rep in ((0.7, 40, 0.9, 1.3), (0.7, 0, 1.0, 1.3), (1.0, 0, 0.8, 1.3), (0.7, 0, 0.8, 1.0)):
+        p = SamplingC(temp, top_k, top_p, 0.0, rep, 0.0, 0.1 * (rep != 1.0), 0)
+        got = []
+        for own in (False, True):
+            src = l.clone()
+            dst = src if own else torch.empty_like(src)
+            tok = torch.empty(1, dtype=torch.int32, device="cuda")
+            call("smx_sample", src.data_ptr(), n, ctx.data_ptr(), ctx.numel(), ctypes.byref(p), 0.37, dst.data_ptr(),
+                 tok.data_ptr(), torch.cuda.current_stream().cuda_stream)
+            got.append((int(tok.item()), dst))
+        assert got[0][0] == got[1][0], (temp, top_k, top_p, rep)
+        assert torch.equal(got[0][1], got[1][1]), (temp, top_k, top_p, rep)
+
+
 def test_stream_read_runs_and_checks_its_size(gpu):
     """smx_stream_read (the bench's streaming-read ceiling) reads device memory without writing
     it, and refuses sizes that are not a positive multiple of 16 bytes."""
