@@ -423,23 +423,34 @@ int fmt_from_type(int type)
     }
 }
 
+// Elements per launch of a codec: at four per thread, half of the 2^32 threads above which a launch does
+// not run them all.
+constexpr int64_t kLaunchElems = (int64_t)1 << 33;
+
 hipError_t launch_dequant_gguf(int type, const void *blocks, int64_t n, float *out, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    const dim3 grid(grid_for((n + 3) / 4));
     return by_type(type, [&](auto t) {
-        hipLaunchKernelGGL((k_dequant_gguf<decltype(t)::value>), grid, dim3(kThreads), 0, s, (const uint8_t *)blocks, n,
-                           out);
+        constexpr int T = decltype(t)::value;
+        for (int64_t e = 0; e < n; e += kLaunchElems) {
+            const int64_t m = n - e < kLaunchElems ? n - e : kLaunchElems;
+            hipLaunchKernelGGL((k_dequant_gguf<T>), dim3(grid_for((m + 3) / 4)), dim3(kThreads), 0, s,
+                               (const uint8_t *)blocks + e / Type<T>::elems * Type<T>::bytes, m, out + e);
+        }
     });
 }
 
 hipError_t launch_quantize_gguf(int type, const float *x, int64_t n, void *blocks, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    const dim3 grid(grid_for((n + 3) / 4));
     return by_type(type, [&](auto t) {
-        if constexpr (decltype(t)::value != SMX_TYPE_F32)
-            hipLaunchKernelGGL((k_quantize<decltype(t)::value>), grid, dim3(kThreads), 0, s, x, n, (uint8_t *)blocks);
+        constexpr int T = decltype(t)::value;
+        if constexpr (T != SMX_TYPE_F32)
+            for (int64_t e = 0; e < n; e += kLaunchElems) {
+                const int64_t m = n - e < kLaunchElems ? n - e : kLaunchElems;
+                hipLaunchKernelGGL((k_quantize<T>), dim3(grid_for((m + 3) / 4)), dim3(kThreads), 0, s, x + e, m,
+                                   (uint8_t *)blocks + e / Type<T>::elems * Type<T>::bytes);
+            }
     });
 }
 

@@ -101,6 +101,35 @@ def test_codecs_at_any_alignment(gpu, name, nblocks):
     assert np.array_equal(got[1:-1], O.quantize(qt, x[1:])) and got[0] == got[-1] == 0xA5
 
 
+@pytest.mark.parametrize("name", ["Q4_K", "Q8_0"])
+def test_codecs_beyond_one_launch(gpu, name):
+    """More elements than one launch takes (2^34 and a few blocks: four per thread, and a launch of more
+    than 2^32 threads does not run them all, without an error): the blocks and floats at the start, at multiples of 2^32 elements and at the
+    end are those of the same elements by themselves."""
+    import torch
+
+    from smallmind_amd.quantization import dequantize, quantize
+    qt = ALL_TYPES[name]
+    n, part = 2 ** 34 + 768, 1024
+    if torch.cuda.mem_get_info()[0] < 160 * 2 ** 30:
+        pytest.skip("needs 160 GiB of free device memory")
+    at = [k * 2 ** 32 + d for k in range(4) for d in (0, 2 ** 32 - part)] + [n - part]
+    x = torch.zeros(n, device="cuda")
+    for i, e in enumerate(at):
+        x[e:e + part] = torch.randn(part, device="cuda", generator=torch.Generator("cuda").manual_seed(i))
+    blocks = quantize(qt, x)
+    per = O.BLOCK_BYTES[qt], O.BLOCK_ELEMS[qt]
+    few = [quantize(qt, x[e:e + part].clone()) for e in at]
+    for e, b in zip(at, few):
+        assert torch.equal(blocks[e // per[1] * per[0]:(e + part) // per[1] * per[0]], b), e
+    del x
+    y = dequantize(qt, blocks, n)
+    for e, b in zip(at, few):
+        assert torch.equal(y[e:e + part], dequantize(qt, b, part)), e
+    del y, blocks
+    torch.cuda.empty_cache()
+
+
 def test_fill_normal_statistics(gpu):
     from smallmind_amd.quantization import fill_normal
     v = fill_normal(5, 1_000_001, 0.02).cpu().numpy().astype(np.float64)
