@@ -927,13 +927,25 @@ __device__ __forceinline__ void unpack8(const float4 &a, const float4 &b, float 
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
+// Sub-block sums of the values of item i of token m (the items of a sub-block are four neighbouring lanes).
+template <int SUMS>
+__device__ __forceinline__ void qprep_sums(const float *v, uint8_t *xp, int nsb, int m, int Mp, int i)
+{
+    if constexpr (SUMS != 0) {
+        float q = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+        q += __shfl_xor(q, 1, 64);
+        const float o = __shfl_xor(q, 2, 64);
+        if ((i & 3) == 0) xp_sums(xp, SUMS, Mp, nsb, m, i >> 2, q, o);
+    }
+}
+
 // One workgroup per token (rows M..Mp-1 of the last tile are zero): the norm statistic of the
 // row (RMSNorm: RMSNormOps.cs:114; LayerNorm: LayerNormOps.cs:92-119), the normalised value in
 // the reference's operation order (gamma * (x * invRms); fma(gamma, (x - mean) * invStd, beta)),
 // then its three bf16 parts at Xp[m/16][s][p][g][m%16][perm].  Thread j holds items j + 256 u
 // (u < IPT, K <= 2048 * IPT): the row, gamma and beta are loaded in one batch before the
-// statistic, so the kernel makes one round trip to memory.
-template <int IPT>
+// statistic, so the kernel makes one round trip to memory.  SUMS: the kind of sub-block sums written (xp_sums).
+template <int IPT, int SUMS>
 __global__ __launch_bounds__(256) void k_qprep(const float *__restrict__ x, int64_t x_stride, int M, int K,
                                                int pro, const float *__restrict__ gamma,
                                                const float *__restrict__ beta, float eps,
@@ -947,7 +959,10 @@ __global__ __launch_bounds__(256) void k_qprep(const float *__restrict__ x, int6
     const int tid = threadIdx.x;
     if (m >= M) {   // padding row of the last tile
         float z[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        for (int i = tid; i < items; i += 256) qprep_store(z, xp, nsb, tt, t, i);
+        for (int i = tid; i < items; i += 256) {
+            qprep_store(z, xp, nsb, tt, t, i);
+            qprep_sums<SUMS>(z, xp, nsb, m, (int)gridDim.x, i);
+        }
         return;
     }
     float4 xa[IPT][2], ga[IPT][2], ba[IPT][2];
@@ -1022,10 +1037,12 @@ __global__ __launch_bounds__(256) void k_qprep(const float *__restrict__ x, int6
             for (int k = 0; k < 8; k++) v[k] = __builtin_fmaf(gg[k], (v[k] - mean) * sc, be[k]);
         }
         qprep_store(v, xp, nsb, tt, t, i);
+        qprep_sums<SUMS>(v, xp, nsb, m, (int)gridDim.x, i);
     }
 }
 
 // Rows longer than 2048 * 4: the same with the row read twice in loops.
+template <int SUMS>
 __global__ __launch_bounds__(256) void k_qprep_long(const float *__restrict__ x, int64_t x_stride, int M, int K,
                                                     int pro, const float *__restrict__ gamma,
                                                     const float *__restrict__ beta, float eps,
@@ -1088,10 +1105,11 @@ __global__ __launch_bounds__(256) void k_qprep_long(const float *__restrict__ x,
             for (int k = 0; k < 8; k++) v[k] = 0.0f;
         }
         qprep_store(v, xp, nsb, tt, t, i);
+        qprep_sums<SUMS>(v, xp, nsb, m, (int)gridDim.x, i);
     }
 }
 
-// More than 16 tokens, or no norm: a workgroup takes 4 tokens (a quarter of a token tile), thread (item lane
+// Many tokens (qprep_per_token), or no norm: a workgroup takes 4 tokens (a quarter of a token tile), thread (item lane
 // tid / 4, token tid % 4).  Four neighbouring lanes store the same item of four tokens, 64
 // contiguous bytes of a part (one token per workgroup stored 16-byte pieces 256 bytes apart, which
 // ran at a third of the copy rate).  The rows of a norm are read again from the L1 for the
@@ -1350,6 +1368,58 @@ hipError_t launch_qgemm_tile(const QgemmArgs &a, hipStream_t s)
     }
 }
 
+namespace {
+
+// Under a norm, up to these many tokens a workgroup per token, which holds its row in registers; above, the
+// store pattern of k_qprep_tokens counts for more.  Per token / four tokens, us, RMSNorm: K 768 17 tokens
+// 2.5 / 3.1, 256 3.4 / 3.4, 320 3.8 / 3.4; K 2048 3.0 / 4.6, 5.0 / 5.1, 5.8 / 5.2; K 5632 4.8 / 8.6, 9.1 / 9.6,
+// 11.2 / 10.1.  LayerNorm, which reads the row once more: K 768 17 tokens 3.0 / 3.9, 320 4.2 / 4.2, 384
+// 4.5 / 4.3; K 2048 3.5 / 6.1, 6.4 / 6.6, 6.8 / 6.7.
+bool qprep_per_token(int M, int pro) { return pro != PRO_NONE && M <= (pro == PRO_LN ? 320 : 256); }
+
+template <int SUMS>
+hipError_t launch_qprep_k(const QgemmArgs &a, const float *x, int64_t x_stride, int pro, const float *gamma,
+                          const float *beta, float eps, hipStream_t s)
+{
+    const int K = (int)a.w.cols;
+    const unsigned mp = (unsigned)((a.M + 15) / 16 * 16);
+    uint8_t *xp = (uint8_t *)a.xp;
+    if (qprep_per_token(a.M, pro)) {
+        const auto run = [&](auto *kernel) {
+            hipLaunchKernelGGL(kernel, dim3(mp), dim3(256), 0, s, x, x_stride, a.M, K, pro, gamma, beta, eps, xp);
+        };
+        switch ((K / 8 + 255) / 256) {
+        case 1: run(k_qprep<1, SUMS>); break;
+        case 2: run(k_qprep<2, SUMS>); break;
+        case 3: run(k_qprep<3, SUMS>); break;
+        case 4: run(k_qprep<4, SUMS>); break;
+        default: run(k_qprep_long<SUMS>); break;
+        }
+    } else {
+        const unsigned span = qprep_span(mp / 4, K / 8, pro);
+        const auto run = [&](auto *kernel) {
+            hipLaunchKernelGGL(kernel, dim3(mp / 4, (K / 8 + span - 1) / span), dim3(256), 0, s, x, x_stride, a.M, K,
+                               gamma, beta, eps, xp, (int)span);
+        };
+        if (pro == PRO_NONE) run(k_qprep_tokens<PRO_NONE, SUMS>);
+        else if (pro == PRO_RMS) run(k_qprep_tokens<PRO_RMS, SUMS>);
+        else run(k_qprep_tokens<PRO_LN, SUMS>);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_qprep(const QgemmArgs &a, const float *x, int64_t x_stride, int pro, const float *gamma,
+                        const float *beta, float eps, hipStream_t s)
+{
+    switch (qgemm_sums_kind(a.w, a.M)) {
+    case 0: return launch_qprep_k<0>(a, x, x_stride, pro, gamma, beta, eps, s);
+    case 1: return launch_qprep_k<1>(a, x, x_stride, pro, gamma, beta, eps, s);
+    default: return launch_qprep_k<2>(a, x, x_stride, pro, gamma, beta, eps, s);
+    }
+}
+
+}  // namespace
+
 hipError_t launch_qgemm(const QgemmArgs &a, const float *x, int64_t x_stride, int pro,
                         const float *gamma, const float *beta, float eps, hipStream_t s)
 {
@@ -1366,33 +1436,10 @@ hipError_t launch_qgemm(const QgemmArgs &a, const float *x, int64_t x_stride, in
     if ((a.rss || a.np) && (a.M > 16 || K % 256 != 0 || fmt_dense(a.w.fmt))) return hipErrorInvalidValue;
     if (a.rss && (x || pro != PRO_NONE || a.rss_n < 1 || a.rss_n > 256)) return hipErrorInvalidValue;
     if (a.np && (a.epi != EPI_RESID || a.w.rows % 32 != 0 || !a.ngamma || !a.nss)) return hipErrorInvalidValue;
-    const unsigned mp = (unsigned)((a.M + 15) / 16 * 16);
-    int ipt = (K / 8 + 255) / 256;
-#define SMX_QPREP(KN) hipLaunchKernelGGL(KN, dim3(mp), dim3(256), 0, s, x, x_stride, a.M, K, pro, gamma, beta, eps, (uint8_t *)a.xp)
-    const unsigned span = qprep_span(mp / 4, K / 8, pro);
-#define SMX_QPREPT(P, S) hipLaunchKernelGGL((k_qprep_tokens<P, S>), dim3(mp / 4, (K / 8 + span - 1) / span), dim3(256), 0, s, x, x_stride, a.M, K, gamma, beta, eps, (uint8_t *)a.xp, (int)span)
-    if (!x) ipt = -1;   // the parts are already in a.xp (written by the producing kernel)
-    if (x && (a.M > 16 || pro == PRO_NONE)) {
-        const int kind = qgemm_sums_kind(a.w, a.M);
-#define SMX_QPREPP(P) do { if (kind == 0) SMX_QPREPT(P, 0); else if (kind == 1) SMX_QPREPT(P, 1); else SMX_QPREPT(P, 2); } while (0)
-        if (pro == PRO_NONE) SMX_QPREPP(PRO_NONE);
-        else if (pro == PRO_RMS) SMX_QPREPP(PRO_RMS);
-        else SMX_QPREPP(PRO_LN);
-#undef SMX_QPREPP
-        ipt = -1;
+    if (x) {   // (else the parts are already in a.xp, written by the producing kernel)
+        const hipError_t e = launch_qprep(a, x, x_stride, pro, gamma, beta, eps, s);
+        if (e != hipSuccess) return e;
     }
-    switch (ipt) {
-    case -1: break;
-    case 1: SMX_QPREP(k_qprep<1>); break;
-    case 2: SMX_QPREP(k_qprep<2>); break;
-    case 3: SMX_QPREP(k_qprep<3>); break;
-    case 4: SMX_QPREP(k_qprep<4>); break;
-    default: SMX_QPREP(k_qprep_long); break;
-    }
-#undef SMX_QPREP
-#undef SMX_QPREPT
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
     if (qgemm_tiled(a.w, a.M)) return launch_qgemm_tile(a, s);
     switch (a.w.fmt) {
     case FMT_Q4_0: return launch_f<FMT_Q4_0>(a, s);

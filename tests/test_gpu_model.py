@@ -296,6 +296,48 @@ def test_forward_api_matches_nocache_reference(pairs, key):
     sess.close()
 
 
+def _prompt_error(cfg, types, tokens, seed=3):
+    """Largest logits error of prompts of these lengths (one prefill chunk each), relative to the oracle's
+    largest logit.  types: layers, embedding, head."""
+    om, gm, _ = build_pair(cfg, *types, seed=seed)
+    try:
+        worst = 0.0
+        for n in tokens:
+            prompt = np.random.default_rng(n).integers(0, cfg.vocab_size, n).astype(np.int32)
+            sess, osess = gm.create_session(n + 8), om.session(n + 8)
+            osess.prefill(prompt[:-1], 0)
+            err = rel_err(sess.forward(prompt, 0), osess.step(int(prompt[-1]), n - 1))
+            print(cfg.architecture, types, n, err, flush=True)
+            worst = max(worst, err)
+            sess.close()
+        return worst
+    finally:
+        gm.close()
+
+
+# Prompts on the matrix-core path: activations as three bf16 parts (2^-24) and fp32 sums of up to 8192
+# terms, each side of every product rounded a few dozen times at 2^-24 relative to the sum of magnitudes,
+# over two layers: some 1e-6 to 1e-5 of the largest logit.  A missing or misplaced sub-block sum is an error of
+# the code offset times the activations, 1e-2 and more.
+PROMPT_TOL = 3e-5
+
+
+@pytest.mark.parametrize("arch,fmt,d,heads,kv,ff,tokens", [
+    ("llama", "Q4_0", 256, 4, 2, 8192, (17, 31, 100, 256, 257)),    # sums of every sub-block; RMSNorm
+    ("llama", "Q6_K", 256, 4, 2, 8192, (17, 31, 100, 256, 257)),    # sums of 16 elements
+    ("gpt2", "Q6_K", 1024, 16, 16, 4096, (130, 320, 321)),          # LayerNorm
+    ("gpt2", "Q8_0", 768, 12, 12, 3072, (17, 33, 320, 321)),        # no sums; three rows of a wave
+    ("llama", "Q8_0", 6144, 96, 8, 256, (20,)),                     # three items per thread
+    ("gpt2", "Q8_0", 2304, 36, 36, 9216, (18,)),                    # two, the second partly beyond the row
+])
+def test_prompt_preparation_under_a_norm(gpu, arch, fmt, d, heads, kv, ff, tokens):
+    """The first GEMM after a norm, on both sides of the token counts up to which a workgroup prepares
+    one token (256 with RMSNorm, 320 with LayerNorm) and at partly filled token tiles."""
+    qt = getattr(O, fmt)
+    assert _prompt_error(ModelConfig(arch, 500, 512, d, 2 if d <= 1024 else 1, heads, kv, ff), (qt, O.Q8_0, O.Q8_0),
+                         tokens) <= PROMPT_TOL
+
+
 def test_decode_is_deterministic_and_cache_equals_recompute(pairs):
     om, gm = _pair(pairs, "llama-q4k")
     prompt = np.arange(12, dtype=np.int32) * 7
