@@ -1326,18 +1326,39 @@ size_t qgemm_parts_bytes(int M, int K) { return (size_t)(((int64_t)M + 15) / 16)
 size_t qgemm_xp_bytes(int M, int K) { return qgemm_parts_bytes(M, K) / 16 * 17; }
 
 int64_t qgemm_tiles(const WView &w, int M) { return ((w.rows + 63) / 64) * (((int64_t)M + 63) / 64); }
+int64_t qgemm_tile_groups(const WView &w, int M) { return ((w.rows + 127) / 128) * (((int64_t)M + 31) / 32); }
 
-// With few 64 x 64 tiles the K-split kernel (16 x 16 tiles, up to 8 waves on one tile's K) fills the
-// chip better.  Measured per call, K-split / tile: 2048 x 2048 Q8_0 at 256 tokens (128 tiles) 31 / 34
-// us, at 384 tokens 44 / 36; Q6_K 34 / 39 and 53 / 42; Q4_K at 511 tokens (256 tiles) 38 / 39, 16384 x
-// 2048 at 128 tokens (512) 56 / 51, 2560 x 2048 at 511 (320) 44 / 47, at 700 (440) 54 / 52.  From 640
-// tokens (K-quants with mins, which the K-split kernel runs on larger tiles: 1024) the tile kernel is
-// level or ahead at every row count (768 x 768 at 700 tokens Q8_0 35 / 25, Q4_K at 1024 25 / 26).
+// Both kernels' times go in steps, a round of workgroups over the chip each, so neither wins from one size
+// on.  S: workgroups of the K-split kernel at 32 rows x 64 tokens; G: those of the tile kernel at 128 x 32.
+//  - Q8_0, Q4_0, SMQ, Q6_K: the tile kernel wins as soon as the K-split kernel needs a second round.
+//    That is S > 256 with 8 waves on a tile (few rows or long K, and Q6_K: K-split / tile, us, 2048 x 2048 Q8_0
+//    256 tokens 28 / 34, 320 44 / 35; 5632 x 5632 64 35 / 47, 65 60 / 49) and S > 512 with 4 (2304 x 768 Q8_0 448
+//    24 / 25, 511 28 / 25).  Longer K moves the line down, the products that remove Q4_0's offset move it up.
+//  - Q4_K, Q5_K, whose K-split kernel runs larger tiles: by G, except in the first part of a new step of the
+//    tile kernel (11264 x 2048 Q4_K at 128 tokens 41 / 42, 160 48 / 45, 192 56 / 60, 256 67 / 64, 352 84 / 76, 384
+//    91 / 96, 448 100 / 99, 511 111 / 102; 5632 x 2048 192 35 / 41, 320 47 / 46, 384 55 / 61, 512 67 / 64).
+// Where the two are level, the tile kernel (its sums are the more exact).
 bool qgemm_tiled(const WView &w, int M)
 {
     if (M <= 16 || w.cols % 256 != 0 || fmt_dense(w.fmt)) return false;
-    const bool mins = w.fmt == FMT_Q4_K || w.fmt == FMT_Q5_K;
-    return M >= (mins ? 1024 : 640) || qgemm_tiles(w, M) >= (mins ? 440 : 160);
+    const int64_t N = w.rows, K = w.cols;
+    const int64_t G = qgemm_tile_groups(w, M), S = ((N + 31) / 32) * (((int64_t)M + 63) / 64);
+    const bool tall = N >= 8192, narrow = N <= 2048 || K > 4096;
+    if (w.fmt == FMT_Q4_K || w.fmt == FMT_Q5_K) {
+        if (M <= 32) return false;
+        if (tall && K < 2048) return G >= 400;
+        if (tall) return G >= 390 && !(G > 512 && G <= 640) && !(K < 4096 && G > 1024 && G < 1200);
+        if (narrow && M <= 320) return S > 256;
+        if (N <= 2048) return G >= (M >= 1024 ? 190 : 400);
+        if (G > 512 && G <= (N > 4096 ? 600 : 576)) return false;
+        if (K < 2048 && N > 4096) return G >= 600 && !(G > 1024 && G < 1188);
+        return G >= (K < 2048 ? 475 : K < 4096 ? 420 : 390);
+    }
+    if (M >= 1024 && S > 200) return true;
+    if (w.fmt == FMT_Q6_K || (narrow && (w.fmt != FMT_SQ8 || K >= 2048))) return S > 256;   // (SQ8: 4 waves)
+    if (K >= 4096) return S >= 352;
+    const bool offset = w.fmt == FMT_Q4_0 || w.fmt == FMT_SQ4;
+    return S > (K >= 2048 ? (tall && offset ? 512 : 352) : offset ? 704 : 512);
 }
 
 int qgemm_sums_kind(const WView &w, int M)

@@ -643,22 +643,23 @@ hipError_t launch_tile(const QgemmArgs &a, hipStream_t s)
 #define SMX_CAT2(a, b) a##b
 #define SMX_CAT(a, b) SMX_CAT2(a, b)
 
-// Shapes by the number of 64 x 64 tiles (W) against the chip's 1024 SIMDs, measured (microseconds with
-// k_qprep_tokens, Q8_0 / Q4_K):
-//  - W >= 1024, four waves of 64 x 64 sharing their parts: 11264 x 2048 at 511 tokens 104 / 106
-//    (W 1408; 64 x 32 tiles 112 / 117), 2048 x 5632 at 2048 tokens 175 / 176 (199 / 200);
-//  - 520 < W < 1024, two waves of 64 x 32: 2560 x 2048 at 1024 tokens 64 / 68 (K split in two 69 / 72,
-//    64 x 64 tiles 73 / 79);
-//  - fewer, 64 x 32 tiles with K split in two (2048 x 5632 at 1024 tokens 108 / 107; unsplit 133 /
-//    143), and in four at W <= 256 when every part has two super-blocks (2048 x 8192 at 511 tokens
-//    84 / 90; in two 91 / 97).
+// Shapes by the workgroups of 128 rows x 32 tokens (G), measured (microseconds with k_qprep_tokens, Q8_0 /
+// Q4_K):
+//  - G >= 1024, and where these make exactly one workgroup per CU: four waves of 64 x 64 sharing their parts:
+//    11264 x 2048 at 511 tokens 104 / 106 (G 1408; 64 x 32 tiles 112 / 117), 2048 x 5632 at 2048 tokens 175 / 176
+//    (199 / 200);
+//  - 512 < G < 1024, two waves of 64 x 32, all in one round: 2560 x 2048 at 1024 tokens 64 / 68 (K split in two
+//    69 / 72, 64 x 64 tiles 73 / 79), 11264 x 2048 at 352 tokens Q4_K 76 (64 x 64 tiles, 264 workgroups, 94);
+//  - fewer, 64 x 32 tiles with K split in two, two workgroups per CU (2048 x 5632 at 1024 tokens 108 / 107;
+//    unsplit 133 / 143; 11264 x 2048 at 160 tokens Q4_K 45, unsplit 58), and in four at up to 256 64 x 64 tiles
+//    when every part has two super-blocks (2048 x 8192 at 511 tokens 84 / 90; in two 91 / 97).
 hipError_t SMX_CAT(launch_qgemm_tile_f, SMX_TILE_FMT)(const QgemmArgs &a, hipStream_t s)
 {
     constexpr int F = SMX_TILE_FMT;
-    const int64_t W = qgemm_tiles(a.w, a.M);
-    if (W >= 1024) return launch_tile<F, 4, 1, 2, 2>(a, s);
-    if (W > 520) return launch_tile<F, 2, 1, 1, 2>(a, s);
-    if (W <= 256 && a.w.cols >= 2048) return launch_tile<F, 2, 4, 1, 2>(a, s);
+    const int64_t G = qgemm_tile_groups(a.w, a.M);
+    if (G >= 1024 || ((a.w.rows + 255) / 256) * ((a.M + 63) / 64) == 256) return launch_tile<F, 4, 1, 2, 2>(a, s);
+    if (G > 512) return launch_tile<F, 2, 1, 1, 2>(a, s);
+    if (qgemm_tiles(a.w, a.M) <= 256 && a.w.cols >= 2048) return launch_tile<F, 2, 4, 1, 2>(a, s);
     return launch_tile<F, 2, 2, 1, 2>(a, s);
 }
 

@@ -222,10 +222,11 @@ struct QgemmArgs {
 // sub-block sums behind them.
 size_t qgemm_parts_bytes(int M, int K);
 size_t qgemm_xp_bytes(int M, int K);
-// Whether the GEMM of M tokens with w runs on the tile kernel (k_qgemm_tile.hip), its number of 64 x 64
-// tiles, and which sub-block sums it reads (a kind of xp_sums, 0: none).
+// Whether the GEMM of M tokens with w runs on the tile kernel (k_qgemm_tile.hip), its numbers of 64 x 64
+// tiles and of 128 x 32 workgroups, and which sub-block sums it reads (a kind of xp_sums, 0: none).
 bool qgemm_tiled(const WView &w, int M);
 int64_t qgemm_tiles(const WView &w, int M);
+int64_t qgemm_tile_groups(const WView &w, int M);
 int qgemm_sums_kind(const WView &w, int M);
 // Sub-block sums to write behind activation parts: their kind and the tokens of the whole batch.
 struct XpSums {

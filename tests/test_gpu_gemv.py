@@ -151,7 +151,12 @@ def test_matmul_matrix_core_random_bytes(gpu, name):
                                    (700, 3100, 512),      # two waves of 64 x 32
                                    (517, 3600, 768),      # K split in two: 2 + 1 super-blocks
                                    (1030, 200, 2304),     # K split in four: 3 + 3 + 3 + 0 super-blocks
-                                   (641, 70, 2048)])      # few rows, many tokens
+                                   (641, 70, 2048),       # few rows, many tokens (the K-split kernel)
+                                   # the K-quants with mins reach the same shapes at these sizes
+                                   (1313, 4100, 256), (1300, 4160, 768),
+                                   (1030, 800, 2304),     # K split in four, the last part empty
+                                   (6101, 70, 2048),      # few rows on the tile kernel
+                                   (195, 16300, 256)])    # one workgroup of four waves per CU
 def test_matmul_tile_kernel_vs_float64(gpu, name, m, N, K):
     """The tile kernel (long prompts) at the edges of its tiles and K splits, on random bytes (every
     code, scale and min value, fp16 scales of any magnitude) and rows of very different size.  Bound
@@ -171,15 +176,16 @@ def test_matmul_tile_kernel_vs_float64(gpu, name, m, N, K):
     assert worst <= 1.0, worst
 
 
-@pytest.mark.parametrize("name,m,K", [("Q8_0", 5, 544),     # one span of 64 eight-element items and one of 4
-                                      ("Q4_0", 16, 4128),   # nine spans, the last of 4 items
-                                      ("Q5_K", 13, 8448),   # padding tokens in the last group of four
-                                      ("Q4_K", 2500, 2304),  # spans of 128 items with sub-block sums, the last of 32
-                                      ("Q6_K", 2500, 2304)])  # the same with sums of half sub-blocks
-def test_matmul_activation_spans_vs_float64(gpu, name, m, K):
+@pytest.mark.parametrize("name,m,N,K", [("Q8_0", 5, 40, 544),     # one span of 64 eight-element items and one of 4
+                                        ("Q4_0", 16, 40, 4128),   # nine spans, the last of 4 items
+                                        ("Q5_K", 13, 40, 8448),   # padding tokens in the last group of four
+                                        ("Q4_K", 2500, 40, 2304),   # spans of 128 items, the last of 32
+                                        ("Q4_K", 2500, 400, 2304),  # the same with sub-block sums
+                                        ("Q6_K", 2500, 400, 2304)])  # with sums of half sub-blocks
+def test_matmul_activation_spans_vs_float64(gpu, name, m, N, K):
     """Activation parts written by several workgroups per row, at ragged last spans; the GEMM bound
     of this file per output."""
-    qt, N = TYPES[name], 40
+    qt = TYPES[name]
     W = quantized(qt, (N, K), seed=m + K)
     X = np.random.default_rng(m + K).normal(0, 1, (m, K)).astype(np.float32)
     Y = _dev(_gemv(qt, W, N, K, X, m=m)).double()
