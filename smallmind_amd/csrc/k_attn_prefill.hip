@@ -746,12 +746,6 @@ __global__ __launch_bounds__(kFewWaves * 64) void k_attn_prefill_few(
 
 constexpr int kRW = 4, kKW = 2;      // k_attn_prefill: 128 rows per workgroup, keys split in two
 
-// Whether `rows` query rows (tokens x heads) fill the chip as 128-row workgroups.  Below about 100 of
-// them the chain of keys of each counts and the 32-row kernel is faster.  Measured (us, 32-row /
-// 128-row): 32 / 4 heads, 511 tokens (128 workgroups) 51 / 41, 32 / 8 heads, 700 tokens at 500 .. (176)
-// 147 / 90; 32 / 32 heads, 255 tokens (64) 21 / 28; 32 / 4 heads, 40 tokens at 1000 .. (10) 49 / 77.
-bool many_rows(int64_t rows) { return rows >= 100 * 32 * kRW; }
-
 }  // namespace
 
 bool attention_prefill_supported(int n_head, int n_kv_head, int hd)
@@ -781,10 +775,23 @@ hipError_t launch_prefill(unsigned blocks, const float *q, int q_stride, const f
     return hipGetLastError();
 }
 
-// tokens per workgroup of the kernel that runs `tokens` tokens
-int attention_prefill_block_rows(int n_head, int n_kv_head, int tokens)
+// 128-row workgroups where the query rows (tokens x heads) would fill 100 of them and every run is long
+// enough that they replace at least twice as many 32-row ones.  With fewer rows the chain of keys of each
+// workgroup counts.  Measured (us, 32-row / 128-row): 32 / 4 heads, 511 tokens (128 workgroups) 51 / 41, 32 / 8
+// heads, 700 tokens at 500 .. (176) 147 / 90; 32 / 32 heads, 255 tokens (64) 21 / 28; 32 / 4 heads, 40 tokens at
+// 1000 .. (10) 49 / 77.  Short runs leave most of a 128-row workgroup empty: 32 / 32 heads, 24 runs of 20 tokens
+// 24 / 34 (768 workgroups either way), of 32 30 / 35, of 33 (1536 / 768) 41 / 35; 64 of 16 46 / 89.
+PrefillPlan attention_prefill_plan(int n_head, int n_kv_head, const int *counts, int n)
 {
-    return (many_rows((int64_t)tokens * n_head) ? 32 * kRW : kFewRows) / (n_head / n_kv_head);
+    const int few = kFewRows / (n_head / n_kv_head), many = 32 * kRW / (n_head / n_kv_head);
+    int64_t tokens = 0, n_few = 0, n_many = 0;
+    for (int i = 0; i < n; i++) {
+        tokens += counts[i];
+        n_few += (counts[i] + few - 1) / few;
+        n_many += (counts[i] + many - 1) / many;
+    }
+    const bool m = tokens * n_head >= 100 * 32 * kRW && n_few >= 2 * n_many;
+    return {m, m ? many : few};
 }
 
 hipError_t launch_attention_prefill(const float *q, int q_stride, const float *kc, const float *vc, float *out,
@@ -795,9 +802,9 @@ hipError_t launch_attention_prefill(const float *q, int q_stride, const float *k
     if (!attention_prefill_supported(n_head, n_kv_head, hd) || M <= 0 || p_first < 0 || ((n_head * hd) & 31) ||
         p_first + M > ctx_stride || (q_stride & 3) || (out_stride & 3) || tok_off < 0)
         return hipErrorInvalidValue;
-    const int TT = attention_prefill_block_rows(n_head, n_kv_head, M);
-    const unsigned blocks = (unsigned)((M + TT - 1) / TT);
-    return many_rows((int64_t)M * n_head)
+    const PrefillPlan plan = attention_prefill_plan(n_head, n_kv_head, &M, 1);
+    const unsigned blocks = (unsigned)((M + plan.rows - 1) / plan.rows);
+    return plan.many
                ? launch_prefill<true>(blocks, q, q_stride, kc, vc, out, out_stride, n_head, n_kv_head, ctx_stride, p_first,
                                       M, s, out_parts, tok_off, sums, PrefillBlocks{})
                : launch_prefill<false>(blocks, q, q_stride, kc, vc, out, out_stride, n_head, n_kv_head, ctx_stride, p_first,
@@ -805,14 +812,14 @@ hipError_t launch_attention_prefill(const float *q, int q_stride, const float *k
 }
 
 hipError_t launch_attention_prefill_blocks(const float *q, int q_stride, float *out, int out_stride, int n_head,
-                                           int n_kv_head, int hd, int ctx_stride, int n_blocks, int tokens,
+                                           int n_kv_head, int hd, int ctx_stride, int n_blocks, bool many,
                                            const PrefillBlocks &pb, hipStream_t s, uint8_t *out_parts, XpSums sums)
 {
-    if (!attention_prefill_supported(n_head, n_kv_head, hd) || n_blocks <= 0 || tokens < n_blocks || !pb.blk ||
-        !pb.kc_tok || !pb.vc_tok || !pb.pos || ((n_head * hd) & 31) || (q_stride & 3) || (out_stride & 3))
+    if (!attention_prefill_supported(n_head, n_kv_head, hd) || n_blocks <= 0 || !pb.blk || !pb.kc_tok ||
+        !pb.vc_tok || !pb.pos || ((n_head * hd) & 31) || (q_stride & 3) || (out_stride & 3))
         return hipErrorInvalidValue;
     const unsigned blocks = (unsigned)n_blocks;
-    return many_rows((int64_t)tokens * n_head)
+    return many
                ? launch_prefill<true>(blocks, q, q_stride, nullptr, nullptr, out, out_stride, n_head, n_kv_head, ctx_stride,
                                       0, 0, s, out_parts, 0, sums, pb)
                : launch_prefill<false>(blocks, q, q_stride, nullptr, nullptr, out, out_stride, n_head, n_kv_head, ctx_stride,

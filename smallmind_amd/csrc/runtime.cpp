@@ -571,10 +571,10 @@ struct PrefillRun {
 // Runs tokens 0..M-1 of B (ids, pos, kc, vc filled on the device) through every layer on the
 // matrix-core GEMM path, writing K/V into each token's cache; the final norm + head run on rows
 // head_from..M-1 into B.logits.  Same graph as enqueue_step, per token.
-// With n_blk > 0, B.blk holds the runs split into attention blocks (attention_prefill_blocks),
-// and the prefill attention of all runs is one launch per layer.
+// With n_blk > 0, B.blk holds the runs split into attention blocks (attention_prefill_plan, blk_many is
+// its kernel), and the prefill attention of all runs is one launch per layer.
 int run_tokens(const smx_model *m, TokBatch &B, int M, int ctx_stride, int head_from, hipStream_t s,
-               const PrefillRun *run, int n_run = 1, int n_blk = 0)
+               const PrefillRun *run, int n_run = 1, int n_blk = 0, bool blk_many = false)
 {
     const smx_model_config &c = m->cfg;
     const int d = c.d_model, hd = m->hd, Hkv = c.n_kv_head;
@@ -639,8 +639,8 @@ int run_tokens(const smx_model *m, TokBatch &B, int M, int ctx_stride, int head_
         uint8_t *att_xp = att_parts ? B.xp2 : nullptr;
         if (run && n_blk > 0 && attention_prefill_supported(c.n_head, Hkv, hd)) {
             const PrefillBlocks pb{B.blk, B.kc, B.vc, B.pos, layer_off};
-            SMX_HIP(launch_attention_prefill_blocks(B.q, m->nqkv, B.att, d, c.n_head, Hkv, hd, ctx_stride, n_blk, M,
-                                                    pb, s, att_xp, sums));
+            SMX_HIP(launch_attention_prefill_blocks(B.q, m->nqkv, B.att, d, c.n_head, Hkv, hd, ctx_stride, n_blk,
+                                                    blk_many, pb, s, att_xp, sums));
         } else if (run && attention_prefill_supported(c.n_head, Hkv, hd)) {
             for (int i = 0; i < n_run; i++) {
                 const PrefillRun &r = run[i];
@@ -817,8 +817,13 @@ int prefill_sessions(smx_model *m, TokBatch &P, smx_session *const *sessions, in
     auto flush = [&]() -> int {
         if (M == 0) return SMX_OK;
         int nb = 0;
+        bool many = false;
         if (blocks && runs.size() > 1) {
-            const int TB = attention_prefill_block_rows(c.n_head, c.n_kv_head, M);
+            std::vector<int> counts;
+            for (const PrefillRun &r : runs) counts.push_back(r.count);
+            const PrefillPlan plan = attention_prefill_plan(c.n_head, c.n_kv_head, counts.data(), (int)counts.size());
+            const int TB = plan.rows;
+            many = plan.many;
             for (const PrefillRun &r : runs)
                 for (int t = 0; t < r.count; t += TB) {
                     blk[(size_t)(2 * nb)] = r.row0 + t;
@@ -832,7 +837,7 @@ int prefill_sessions(smx_model *m, TokBatch &P, smx_session *const *sessions, in
         SMX_HIP(hipMemcpyAsync(P.kc, kc.data(), (size_t)M * sizeof(float *), hipMemcpyHostToDevice, s));
         SMX_HIP(hipMemcpyAsync(P.vc, vc.data(), (size_t)M * sizeof(float *), hipMemcpyHostToDevice, s));
         SMX_HIP(hipMemcpyAsync(P.tok_arr, ta.data(), (size_t)M * sizeof(int32_t *), hipMemcpyHostToDevice, s));
-        const int rc = run_tokens(m, P, M, ctx_stride, M, s, runs.data(), (int)runs.size(), nb);
+        const int rc = run_tokens(m, P, M, ctx_stride, M, s, runs.data(), (int)runs.size(), nb, many);
         if (rc != SMX_OK) return rc;
         // the host arrays are reused by the next chunk: let this chunk's copies finish
         SMX_HIP(hipStreamSynchronize(s));

@@ -323,8 +323,8 @@ hipError_t launch_attention_prefill(const float *q, int q_stride, const float *k
                                     int p_first, int M, hipStream_t s, uint8_t *out_parts = nullptr,
                                     int tok_off = 0, XpSums sums = XpSums{});
 // Several sessions' runs of a token batch in one launch: workgroup b takes the rows
-// blk[2b] .. blk[2b] + blk[2b+1] - 1 of the batch (at most attention_prefill_block_rows rows of a batch
-// of `tokens` rows, all of one run), with that session's cache (kc_tok / vc_tok of its first row, plus layer_off) and
+// blk[2b] .. blk[2b] + blk[2b+1] - 1 of the batch (at most as many as the plan for the runs says, all of one
+// run), with that session's cache (kc_tok / vc_tok of its first row, plus layer_off) and
 // the first row's position; q, out and the parts are addressed by batch row.
 struct PrefillBlocks {
     const int32_t *blk;
@@ -332,9 +332,14 @@ struct PrefillBlocks {
     const int32_t *pos;
     int64_t layer_off;
 };
-int attention_prefill_block_rows(int n_head, int n_kv_head, int tokens);
+// Tokens per workgroup for runs of these lengths, and whether that is the kernel for many rows.
+struct PrefillPlan {
+    bool many;
+    int rows;
+};
+PrefillPlan attention_prefill_plan(int n_head, int n_kv_head, const int *counts, int n);
 hipError_t launch_attention_prefill_blocks(const float *q, int q_stride, float *out, int out_stride, int n_head,
-                                           int n_kv_head, int hd, int ctx_stride, int n_blocks, int tokens,
+                                           int n_kv_head, int hd, int ctx_stride, int n_blocks, bool many,
                                            const PrefillBlocks &pb, hipStream_t s, uint8_t *out_parts = nullptr,
                                            XpSums sums = XpSums{});
 hipError_t launch_attention_tokens(const float *q, int64_t q_stride, float *const *kc_tok,

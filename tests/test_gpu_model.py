@@ -338,6 +338,29 @@ def test_prompt_preparation_under_a_norm(gpu, arch, fmt, d, heads, kv, ff, token
                          tokens) <= PROMPT_TOL
 
 
+@pytest.mark.parametrize("kv,lens", [(32, range(18, 42)),      # 32-row workgroups: 128-row ones would be a quarter full
+                                     (32, range(60, 84)),      # 128-row workgroups
+                                     (4, range(18, 42)),       # grouped heads: 16 tokens fill a 128-row workgroup
+                                     (4, (5, 200, 3, 17, 100, 129, 2))])
+def test_packed_prompts_attention(gpu, kv, lens):
+    """Prompts of several sessions prefilled together (one attention launch per layer, blocks cut per
+    session), then the logits of the next token of every session against the oracle."""
+    from smallmind_amd.model import GpuInferenceSession
+    om, gm, _ = build_pair(ModelConfig("llama", 500, 256, 2048, 2, 32, kv, 256), O.Q8_0, O.Q8_0, O.Q8_0, seed=kv)
+    rng = np.random.default_rng(len(lens))
+    prompts = [rng.integers(0, 500, n).astype(np.int32) for n in lens]
+    sess = [gm.create_session(256) for _ in prompts]
+    toks, _ = GpuInferenceSession.generate_greedy_batch(sess, prompts, 1)
+    for i, p in enumerate(prompts):
+        o = om.session(256)
+        o.prefill(p, 0)
+        ref = o.step(int(toks[i][0]), len(p))
+        assert rel_err(sess[i].forward(toks[i][:1], len(p)), ref) <= PROMPT_TOL, (i, len(p))
+    for s in sess:
+        s.close()
+    gm.close()
+
+
 def test_decode_is_deterministic_and_cache_equals_recompute(pairs):
     om, gm = _pair(pairs, "llama-q4k")
     prompt = np.arange(12, dtype=np.int32) * 7
