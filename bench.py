@@ -236,6 +236,25 @@ def mean_attended(wl) -> float:
     return wl.prompt_len + (wl.new_tokens - 1) / 2
 
 
+# Paths that reach a step through different kernels sum in different orders: their logits differ by about
+# 1e-6 of the largest, so two logits closer than this may fall either way.
+TIE_TOL = 1e-4
+
+
+def same_or_near_tie(a, b, logits_at):
+    """Whether two greedy token sequences of one prompt agree: (True, None) if they are equal; where they
+    part at step k, (whether both took one of the two largest of logits_at(k) and these are a near-tie, k)."""
+    import numpy as np
+    diff = np.nonzero(np.asarray(a) != np.asarray(b))[0]
+    if len(diff) == 0:
+        return True, None
+    k = int(diff[0])
+    lg = np.asarray(logits_at(k))
+    top = np.argsort(lg)[::-1][:2]
+    margin = float((lg[top[0]] - lg[top[1]]) / np.abs(lg).max())
+    return margin <= TIE_TOL and {int(a[k]), int(b[k])} == {int(t) for t in top}, k
+
+
 def other_configs():
     """configs[0], [3] and [4] measured on the same build: GPT-2-small Q8_0 decode; LLaMA-1.1B
     Q8_0 with a 4096-token prefill (matrix-core GEMM chunks) then decode at ~4.1K context; and
@@ -308,10 +327,21 @@ def other_configs():
         got.append(b.step(1))
     dt = time.perf_counter() - t0
     b.close()
-    # the batcher's tokens are the lockstep run's (same prompts, same model)
+    # the batcher's tokens are the lockstep run's (same prompts, same model), up to a near-tie of the logits:
+    # its prompts are prefilled one by one and the lockstep run's together, through other kernels
     got = np.concatenate(got, axis=1)
-    out["smollm-1.7b-q5_k"]["continuous_batcher_tokens_match_lockstep"] = bool(
-        np.array_equal(got, toks[:, :got.shape[1]]))
+    parted = []
+    agree = True
+    for i, (x, p) in enumerate(zip(sess, prompts)):
+        def logits_at(k):
+            x.reset_kv_cache()
+            return x.forward(np.concatenate([p, toks[i, :k]]).astype(np.int32), 0)
+        same, k = same_or_near_tie(got[i], toks[i, :got.shape[1]], logits_at)
+        agree = agree and same
+        if k is not None:
+            parted.append([i, k])
+    out["smollm-1.7b-q5_k"]["continuous_batcher_tokens_match_lockstep"] = agree
+    out["smollm-1.7b-q5_k"]["continuous_batcher_near_ties"] = parted
     out["smollm-1.7b-q5_k"]["continuous_batcher_ms_per_step"] = round(dt * 1e3 / n_steps, 4)
     out["smollm-1.7b-q5_k"]["continuous_batcher_tok_s_aggregate"] = round(wl.sessions * n_steps / dt, 1)
     for x in sess:

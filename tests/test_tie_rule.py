@@ -36,6 +36,19 @@ def test_difference_without_a_near_tie_fails():
         _same_tokens_or_near_tie(other, ref, _logits(8, 20, tie_at=5, margin=TIE_TOL * 2))
 
 
+@pytest.mark.parametrize("margin,token,agree", [(TIE_TOL / 2, 7, True), (TIE_TOL * 2, 7, False),
+                                                (TIE_TOL / 2, 11, False)])
+def test_bench_rule(margin, token, agree):
+    """bench.py's comparison of two runs: equal, or parted at a near-tie between its two tokens."""
+    from bench import same_or_near_tie
+    ref, lg = np.full(8, 3), _logits(8, 20, tie_at=5, margin=margin)
+    other = ref.copy()
+    assert same_or_near_tie(other, ref, lg.__getitem__) == (True, None)
+    other[5:] = token
+    assert same_or_near_tie(other, ref, lg.__getitem__) == (agree, 5)
+    assert same_or_near_tie(ref, other, lg.__getitem__) == (agree, 5)
+
+
 def test_difference_to_a_token_other_than_the_runner_up_fails():
     ref = np.full(8, 3)
     other = ref.copy()
