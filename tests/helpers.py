@@ -58,8 +58,11 @@ def model_specs(cfg, layer_type, embd_type, head_type):
     return tensor_specs(cfg, layer_type, embd_type, head_type)
 
 
-def build_pair(cfg, layer_type, embd_type, head_type, seed=1234, random_norms=True, with_gpu=True):
-    """Returns (oracle_model, gpu_model or None, {name: (qtype, dims, host bytes)})."""
+def build_pair(cfg, layer_type, embd_type, head_type, seed=1234, random_norms=True, with_gpu=True, types=None,
+               change=None):
+    """Returns (oracle_model, gpu_model or None, {name: (qtype, dims, host bytes)}).  types: {part of a
+    matrix's name: its type} instead of layer_type; change(name, values): edits the values of a tensor before
+    they are encoded."""
     rng = np.random.default_rng(seed)
     arch = O.ARCH_GPT2 if cfg.architecture == "gpt2" else O.ARCH_LLAMA
     om = O.OracleModel(arch, cfg.vocab_size, cfg.context_length, cfg.embedding_length,
@@ -71,6 +74,7 @@ def build_pair(cfg, layer_type, embd_type, head_type, seed=1234, random_norms=Tr
         gm = GpuTransformerModel(cfg)
     tensors = {}
     for s in model_specs(cfg, layer_type, embd_type, head_type):
+        qtype = next((q for part, q in (types or {}).items() if part in s.name), s.qtype)
         if s.kind == "norm":
             data = (rng.normal(1.0, 0.1, s.n) if random_norms else np.ones(s.n)).astype(np.float32)
         elif s.kind == "bias0":
@@ -78,11 +82,15 @@ def build_pair(cfg, layer_type, embd_type, head_type, seed=1234, random_norms=Tr
         elif s.kind == "bias":
             data = rng.normal(0.0, 0.02, s.n).astype(np.float32)
         else:
-            data = O.quantize(s.qtype, rng.normal(0.0, 0.02, s.n).astype(np.float32))
-        om.set_tensor(s.name, s.qtype, data, s.n)
+            data = rng.normal(0.0, 0.02, s.n).astype(np.float32)
+        if change is not None:
+            change(s.name, data)
+        if s.kind not in ("norm", "bias0", "bias"):
+            data = O.quantize(qtype, data)
+        om.set_tensor(s.name, qtype, data, s.n)
         if gm is not None:
-            gm.load_tensor(s.name, s.qtype, s.dims, data)
-        tensors[s.name] = (s.qtype, s.dims, data)
+            gm.load_tensor(s.name, qtype, s.dims, data)
+        tensors[s.name] = (qtype, s.dims, data)
     om.finalize()
     if gm is not None:
         gm.finalize()

@@ -296,10 +296,10 @@ def test_forward_api_matches_nocache_reference(pairs, key):
     sess.close()
 
 
-def _prompt_error(cfg, types, tokens, seed=3):
+def _prompt_error(cfg, formats, tokens, seed=3, **kw):
     """Largest logits error of prompts of these lengths (one prefill chunk each), relative to the oracle's
-    largest logit.  types: layers, embedding, head."""
-    om, gm, _ = build_pair(cfg, *types, seed=seed)
+    largest logit.  formats: layers, embedding, head."""
+    om, gm, _ = build_pair(cfg, *formats, seed=seed, **kw)
     try:
         worst = 0.0
         for n in tokens:
@@ -307,7 +307,7 @@ def _prompt_error(cfg, types, tokens, seed=3):
             sess, osess = gm.create_session(n + 8), om.session(n + 8)
             osess.prefill(prompt[:-1], 0)
             err = rel_err(sess.forward(prompt, 0), osess.step(int(prompt[-1]), n - 1))
-            print(cfg.architecture, types, n, err, flush=True)
+            print(cfg.architecture, formats, n, err, flush=True)
             worst = max(worst, err)
             sess.close()
         return worst
@@ -336,6 +336,53 @@ def test_prompt_preparation_under_a_norm(gpu, arch, fmt, d, heads, kv, ff, token
     qt = getattr(O, fmt)
     assert _prompt_error(ModelConfig(arch, 500, 512, d, 2 if d <= 1024 else 1, heads, kv, ff), (qt, O.Q8_0, O.Q8_0),
                          tokens) <= PROMPT_TOL
+
+
+@pytest.mark.parametrize("arch,fmt,heads,kv,ff,tokens,types", [
+    # sums of the down projection's input from the GELU epilogue, of QKV and up from k_qprep_tokens (LayerNorm),
+    # of the O projection's from the 32-row attention
+    ("gpt2", "Q4_0", 16, 16, 4096, (600,), None),
+    ("gpt2", "Q4_K", 16, 16, 4096, (1030,), None),
+    ("gpt2", "Q6_K", 16, 16, 4096, (600,), None),
+    # from the SwiGLU epilogue (RMSNorm); 820 tokens of 16 heads take the 128-row attention
+    ("llama", "Q6_K", 16, 4, 2048, (600, 820), None),
+    ("llama", "Q4_0", 16, 16, 2048, (600, 820), None),
+    ("llama", "Q5_K", 16, 4, 2048, (1030,), None),
+    # gate/up on the K-split kernel, which writes no sums, before a down projection that reads them
+    ("llama", "Q4_K", 16, 4, 1024, (600,), {"ffn_down": "Q6_K"}),
+    ("llama", "Q4_K", 16, 4, 1024, (600,), {"ffn_down": "Q4_0"}),
+    # ... and the other way round: down reads none
+    ("llama", "Q6_K", 16, 4, 1024, (600,), {"ffn_down": "Q8_0"}),
+    # head dimensions of the attention per token: 16 (no sums from it), 32, 128
+    ("llama", "Q4_0", 64, 64, 1024, (600,), None),
+    ("llama", "Q6_K", 64, 8, 1024, (600,), None),
+    ("llama", "Q4_0", 32, 8, 1024, (600,), None),
+    ("llama", "Q6_K", 8, 8, 1024, (600,), None),
+])
+def test_prompt_sums_between_kernels(gpu, arch, fmt, heads, kv, ff, tokens, types):
+    """Every kernel that writes sub-block sums of activations for a tile GEMM, with the GEMM that reads
+    them (d_model 1024), and the pairs that go without: logits of whole prompts against the oracle."""
+    cfg = ModelConfig(arch, 300, 1100, 1024, 2, heads, kv, ff)
+    assert _prompt_error(cfg, (getattr(O, fmt), O.Q8_0, O.Q8_0), tokens,
+                         types={k: getattr(O, v) for k, v in (types or {}).items()}) <= PROMPT_TOL
+
+
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q6_K"])
+def test_prompt_sums_of_fp32_attention(gpu, fmt):
+    """A cached key with an element beyond what bf16 parts hold sends the 128-row attention's workgroups to
+    fp32; the sums that these write for the O projection.  The element meets a query element of exactly 0
+    (zero rows of a signed 8-bit matrix), so the scores are those of the other dimensions."""
+    d, heads = 1024, 16
+
+    def change(name, v):
+        if "attn_qkv.weight" in name:
+            v.reshape(3 * d, d)[64 * 3 + 5] = 0.0          # query element 5 of head 3
+        if "attn_qkv.bias" in name:
+            v[64 * 3 + 5] = 0.0
+            v[d + 64 * 3 + 5] = 3.39e38                    # the key's
+    cfg = ModelConfig("gpt2", 300, 1100, d, 2, heads, heads, 4 * d)
+    assert _prompt_error(cfg, (O.Q8_0, O.Q8_0, O.Q8_0), (820,), types={"attn_output.weight": getattr(O, fmt)},
+                         change=change) <= PROMPT_TOL
 
 
 @pytest.mark.parametrize("kv,lens", [(32, range(18, 42)),      # 32-row workgroups: 128-row ones would be a quarter full

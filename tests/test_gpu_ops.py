@@ -256,7 +256,9 @@ def test_attention_prefill_many_rows_infinities(gpu):
 
 def _sample64(l, ctx, temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, repetition_penalty=1.0, frequency_penalty=0.0,
               repetition_window=0):
-    """Float32 logits stages, float64 probabilities: (probabilities, whether a cutoff lies within rounding)."""
+    """Float32 logits stages, float64 probabilities: one array for every cutoff that rounding allows.  The
+    fp32 sum behind top-p is within 1e-5 of the exact one (of about 1: a tree of depth 16 over expf's 2 ulp and
+    a division), and so is a probability of the min-p threshold; between them they may fall either way."""
     l, f = l.copy(), np.float32
     w = ctx[len(ctx) - min(len(ctx), repetition_window or 256):]
     for t in np.unique(w):
@@ -267,21 +269,20 @@ def _sample64(l, ctx, temperature=1.0, top_k=0, top_p=1.0, min_p=0.0, repetition
     if 0 < top_k < len(l):
         l = np.where(l >= np.sort(l)[len(l) - top_k], l, f(-np.inf))
     e = np.exp(l.astype(np.float64) - l.max())
-    p, near = e / e.sum(), False
+    out = [e / e.sum()]
     if top_p < 1.0:
-        v, c = np.unique(p, return_counts=True)
-        cum = np.cumsum((v * c)[::-1])
-        near |= bool((np.abs(cum - top_p) < 1e-5).any())
-        p = np.where(p >= v[::-1][np.argmax(cum >= top_p)], p, 0.0)
-        p /= p.sum()
+        v, c = np.unique(out[0], return_counts=True)
+        v, cum = v[::-1], np.cumsum((v * c)[::-1])
+        lo, hi = (int(np.argmax(cum >= top_p + d)) if cum[-1] >= top_p + d else len(v) - 1 for d in (-1e-5, 1e-5))
+        out = [np.where(out[0] >= v[i], out[0], 0.0) for i in range(lo, hi + 1)]
+        out = [p / p.sum() for p in out]
     if min_p > 0.0:
-        near |= bool((np.abs(p / (p.max() * min_p) - 1) < 1e-5).any())
-        p = np.where(p < p.max() * min_p, 0.0, p)
-        p /= p.sum()
-    return p, near
+        out = [np.where(p < p.max() * min_p * d, 0.0, p) for p in out for d in (1 - 1e-5, 1, 1 + 1e-5)]
+        out = [p / p.sum() for p in out]
+    return out
 
 
-@pytest.mark.parametrize("n", [1, 63, 1025, 32000, 32768, 32769, 50257, 65536, 65537])
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 4097, 32000, 32768, 32769, 50257, 65536, 65537])
 @pytest.mark.parametrize("data", ["spread", "flat", "ties", "zeros", "masked"])
 def test_sample_paths_vs_float64(gpu, n, data):
     """Values in LDS, in LDS and registers, and in memory; cutoffs found in the list of candidates and
@@ -305,10 +306,10 @@ def test_sample_paths_vs_float64(gpu, n, data):
         for u in (0.0, float(rng.random()), 1.0 - 2.0 ** -40):
             tok, p = sample(_dev(l), u, context=_dev(ctx), **kw)
             p = p.cpu().numpy().astype(np.float64)
-            ref, near = _sample64(l, ctx, **kw)
-            if near:
-                continue
-            assert np.array_equal(p > 0, ref > 0), (kw, (p > 0).sum(), (ref > 0).sum())
+            allowed = _sample64(l, ctx, **kw) if u == 0.0 else allowed
+            same = [ref for ref in allowed if np.array_equal(p > 0, ref > 0)]
+            assert same, (kw, (p > 0).sum(), [(ref > 0).sum() for ref in allowed])
+            ref = same[0]
             assert np.abs(p - ref).max() <= 2 ** -18 * ref.max(), kw
             cdf = np.cumsum(p)
             if u == 0.0:
