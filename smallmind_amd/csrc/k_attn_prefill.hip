@@ -30,9 +30,9 @@
 // Work decomposition.  A workgroup owns 32 RW query rows of one KV head: 32 RW / G tokens x the G
 // query heads that share the KV head (GQA); a wave owns 32 rows.  Tiles of 32 keys are split into
 // parts once per workgroup and shared through LDS (two slots: the next tile is loaded while the
-// current one is multiplied).  KW > 1: KW groups of RW waves take alternate tiles (short prompts,
-// where rows alone do not fill the chip); their maxima, sums and outputs are combined in LDS in a
-// fixed order.  The workgroups with most keys start first.
+// current one is multiplied).  KW groups of RW waves take alternate tiles, which halves the chain of
+// keys of a workgroup; their maxima, sums and outputs are combined in LDS in a fixed order.  The workgroups
+// with most keys start first.  Few rows take another kernel (below).
 //
 // Operands of v_mfma_f32_32x32x16_bf16 (lane l: li = l % 32, h = l / 32; 8 k-values per lane):
 //   S^T = K . Q^T: A = K (key li, dimensions 16 t + 8 h ..), B = Q^T (query li, same dimensions); D
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
         float mx[KW][RW][kKeys], sum[KW][RW][kKeys];
     };
     struct Red {
-        float o[KW > 1 ? KW - 1 : 1][RW][2 * 16][64];
+        float o[KW - 1][RW][2 * 16][64];
     };
     __shared__ __align__(16) uint8_t s_mem[sizeof(Lds)];
     __shared__ int s_large;   // an operand beyond kPartMax
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
         for (int e = 0; e < 8; e++) large = fmaxf(large, fabsf(x[e]));
     };
     if (threadIdx.x == 0) s_large = 0;   // (read after the loops' barriers)
-    static_assert(KW == 1 || sizeof(Red) <= sizeof(uint4) * KW * 2 * 4 * 3 * 2 * kKeys * 2, "outputs reuse the tiles");
+    static_assert(KW > 1 && sizeof(Red) <= sizeof(uint4) * KW * 2 * 4 * 3 * 2 * kKeys * 2, "outputs reuse the tiles");
     Lds &L = *(Lds *)s_mem;
     Red &R = *(Red *)s_mem;
     const int tid = threadIdx.x, lane = tid & 63, wv = wave_id();
@@ -328,9 +328,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
     for (; it1 < it_full; it1++) pass1(it1, std::false_type{});
     for (; it1 < n_it; it1++) pass1(it1, std::true_type{});
     mx = fmaxf(mx, half_other(mx));
-    if constexpr (KW > 1) {
-        if (h == 0) L.mx[kg][rw][li] = mx;
-    }
+    if (h == 0) L.mx[kg][rw][li] = mx;
 
     // ---- pass 2: exponentials, sums and E.V --------------------------------------------------
     // Iteration it multiplies the scores of tile it + 1 while it exponentiates those of tile it, then
@@ -346,11 +344,9 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
     scores(0, s0);
     store_k(1);
     load_k(kg + 2 * KW);
-    if constexpr (KW > 1) {
-        mx = L.mx[0][rw][li];
+    mx = L.mx[0][rw][li];
 #pragma unroll
-        for (int k = 1; k < KW; k++) mx = fmaxf(mx, L.mx[k][rw][li]);
-    }
+    for (int k = 1; k < KW; k++) mx = fmaxf(mx, L.mx[k][rw][li]);
     __syncthreads();
     float sum = 0.0f;
     f32x16 oh[2];   // dimensions 32 dt ..
@@ -436,25 +432,24 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void k_attn_prefill(
         return;
     }
     sum += half_other(sum);
-    if constexpr (KW > 1) {   // the key groups' sums and outputs, added in order by group 0
-        if (h == 0) L.sum[kg][rw][li] = sum;
-        if (kg > 0) {
+    // the key groups' sums and outputs, added in order by group 0
+    if (h == 0) L.sum[kg][rw][li] = sum;
+    if (kg > 0) {
 #pragma unroll
-            for (int dt = 0; dt < 2; dt++)
+        for (int dt = 0; dt < 2; dt++)
 #pragma unroll
-                for (int i = 0; i < 16; i++) R.o[kg - 1][rw][16 * dt + i][lane] = oh[dt][i];
-        }
-        __syncthreads();
-        if (kg > 0) return;
-        sum = L.sum[0][rw][li];
+            for (int i = 0; i < 16; i++) R.o[kg - 1][rw][16 * dt + i][lane] = oh[dt][i];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+    sum = L.sum[0][rw][li];
 #pragma unroll
-        for (int k = 1; k < KW; k++) {
-            sum += L.sum[k][rw][li];
+    for (int k = 1; k < KW; k++) {
+        sum += L.sum[k][rw][li];
 #pragma unroll
-            for (int dt = 0; dt < 2; dt++)
+        for (int dt = 0; dt < 2; dt++)
 #pragma unroll
-                for (int i = 0; i < 16; i++) oh[dt][i] += R.o[k - 1][rw][16 * dt + i][lane];
-        }
+            for (int i = 0; i < 16; i++) oh[dt][i] += R.o[k - 1][rw][16 * dt + i][lane];
     }
     const float inv = 1.0f / sum;
 #pragma unroll

@@ -944,7 +944,7 @@ __device__ __forceinline__ void qprep_sums(const float *v, uint8_t *xp, int nsb,
 // the reference's operation order (gamma * (x * invRms); fma(gamma, (x - mean) * invStd, beta)),
 // then its three bf16 parts at Xp[m/16][s][p][g][m%16][perm].  Thread j holds items j + 256 u
 // (u < IPT, K <= 2048 * IPT): the row, gamma and beta are loaded in one batch before the
-// statistic, so the kernel makes one round trip to memory.  SUMS: the kind of sub-block sums written (xp_sums).
+// statistic, so the kernel makes one round trip to memory.  pro: PRO_RMS or PRO_LN.  SUMS: the kind of sub-block sums written (xp_sums).
 template <int IPT, int SUMS>
 __global__ __launch_bounds__(256) void k_qprep(const float *__restrict__ x, int64_t x_stride, int M, int K,
                                                int pro, const float *__restrict__ gamma,
@@ -972,10 +972,8 @@ __global__ __launch_bounds__(256) void k_qprep(const float *__restrict__ x, int6
         if (i < items) {
             xa[u][0] = ((const float4 *)xr)[2 * i];
             xa[u][1] = ((const float4 *)xr)[2 * i + 1];
-            if (pro != PRO_NONE) {
-                ga[u][0] = ((const float4 *)gamma)[2 * i];
-                ga[u][1] = ((const float4 *)gamma)[2 * i + 1];
-            }
+            ga[u][0] = ((const float4 *)gamma)[2 * i];
+            ga[u][1] = ((const float4 *)gamma)[2 * i + 1];
             if (pro == PRO_LN) {
                 ba[u][0] = ((const float4 *)beta)[2 * i];
                 ba[u][1] = ((const float4 *)beta)[2 * i + 1];
@@ -995,7 +993,7 @@ __global__ __launch_bounds__(256) void k_qprep(const float *__restrict__ x, int6
             }
         ss = block_sum<4>(ss, red);
         sc = 1.0f / sqrtf(ss / (float)K + eps);
-    } else if (pro == PRO_LN) {
+    } else {
         float tsum = 0.0f;
 #pragma unroll
         for (int u = 0; u < IPT; u++)
@@ -1029,7 +1027,7 @@ __global__ __launch_bounds__(256) void k_qprep(const float *__restrict__ x, int6
             unpack8(ga[u][0], ga[u][1], gg);
 #pragma unroll
             for (int k = 0; k < 8; k++) v[k] = gg[k] * (v[k] * sc);
-        } else if (pro == PRO_LN) {
+        } else {
             float gg[8], be[8];
             unpack8(ga[u][0], ga[u][1], gg);
             unpack8(ba[u][0], ba[u][1], be);
@@ -1093,7 +1091,7 @@ __global__ __launch_bounds__(256) void k_qprep_long(const float *__restrict__ x,
                 unpack8(((const float4 *)gamma)[2 * i], ((const float4 *)gamma)[2 * i + 1], gg);
 #pragma unroll
                 for (int k = 0; k < 8; k++) v[k] = gg[k] * (v[k] * sc);
-            } else if (pro == PRO_LN) {
+            } else {
                 float gg[8], be[8];
                 unpack8(((const float4 *)gamma)[2 * i], ((const float4 *)gamma)[2 * i + 1], gg);
                 unpack8(((const float4 *)beta)[2 * i], ((const float4 *)beta)[2 * i + 1], be);

@@ -1,5 +1,5 @@
-// k_qgemm_tile.hip -- quantized GEMM Y[M][N] = X[M][K] . W[N][K]^T on the bf16 matrix cores for more
-// than 16 tokens (prompt chunks, IWeightTensor.MatMul over many rows; NeuralNet.cs:145-298,
+// k_qgemm_tile.hip -- quantized GEMM Y[M][N] = X[M][K] . W[N][K]^T on the bf16 matrix cores for prompts
+// that make enough tiles (qgemm_tiled; IWeightTensor.MatMul over many rows; NeuralNet.cs:145-298,
 // MatMulF32Q8.cs:23-80) and rows of whole 256-element super-blocks.
 //
 // Exactness is that of k_qgemm.hip: integer weight codes in bf16, activations as three bf16
@@ -14,8 +14,8 @@
 // What bounds it: the matrix cores issue three products (hi, mid, lo) per useful one, so the
 // ceiling is a third of the bf16 rate; next come the CU's data paths.  A wave that loads its own
 // activation parts moves 6 bytes per token and k through the CU's 64 B/clk vector-memory path
-// for 32-64 rows of work, which limited the K-split kernel (now up to 16 tokens only) to
-// 15-27 % matrix-core use.  Hence:
+// for 32-64 rows of work, which limits the K-split kernel (k_qgemm.hip: up to 16 tokens, and
+// prompts of few tiles) to 15-27 % matrix-core use.  Hence:
 //   * a wave computes 64 rows x 32 TT tokens (v_mfma_f32_32x32x16_bf16: a lane owns one weight
 //     row per tile, so block scales are decoded by 2 lanes instead of 4);
 //   * WR waves of a workgroup take different rows and share one copy of the parts in LDS, which

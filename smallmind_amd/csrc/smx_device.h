@@ -187,8 +187,8 @@ __device__ __forceinline__ void xp_store(uint8_t *xp, int nsb, int m, int k, flo
     *(uint16_t *)(b + 2048) = (uint16_t)bf16_rne(r2);
 }
 
-// Sums of the activations of sub-block s (32 elements) of token m, from which the GEMM over more
-// than 16 tokens takes its code-offset and min terms.  They are matrix-core operands, stored as
+// Sums of the activations of sub-block s (32 elements) of token m, from which the tile GEMM (qgemm_tiled)
+// takes its code-offset and min terms.  They are matrix-core operands, stored as
 // three bf16 parts behind the parts of all M tokens: kind 1 (one sum per sub-block)
 // [m / 16][s / 8][part][m % 16][s % 8], kind 2 (one per 16 elements) [m / 16][s / 8][part][half]
 // [m % 16][s % 8].

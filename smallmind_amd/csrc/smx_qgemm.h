@@ -1,5 +1,5 @@
-// smx_qgemm.h -- device code shared by the matrix-core GEMM kernels (k_qgemm.hip: up to 16 tokens and
-// rows of 32-element blocks; k_qgemm_tile.hip: more tokens): the bf16 weight operand of each block
+// smx_qgemm.h -- device code shared by the matrix-core GEMM kernels (k_qgemm.hip: up to 16 tokens, prompts
+// of few tiles and rows of 32-element blocks; k_qgemm_tile.hip: the other prompts, qgemm_tiled): the bf16 weight operand of each block
 // format, the activation-part loads, the per-value epilogue, and the direct-to-LDS load.
 #pragma once
 
@@ -240,8 +240,6 @@ template <> struct QW<FMT_Q6_K> {
 
 constexpr uint4 kZero4 = {0u, 0u, 0u, 0u};
 
-// acc + sc * (C - off * sum x) - m * sum x as two fused steps: acc + sc*C - (sc*off + m) * sum x
-// (cs = sc * off + m precomputed per row and sub-block).
 // Activation part p of (token tile tt, sub-block s) for this lane: a wave-uniform base plus the
 // lane's 32-bit byte offset, so each load is one scalar-base instruction with no per-lane
 // 64-bit address arithmetic.
@@ -251,6 +249,8 @@ __device__ __forceinline__ uint4 ld_part(const uint8_t *xp, int tt, int nsb, int
     return *(const uint4 *)(base + lane16);
 }
 
+// acc + sc * (C - off * sum x) - m * sum x as two fused steps: acc + sc*C - (sc*off + m) * sum x
+// (cs = sc * off + m precomputed per row and sub-block).
 __device__ __forceinline__ float accumulate1(float acc, float sc, float cs, float c, float sx)
 {
     return __builtin_fmaf(sc, c, __builtin_fmaf(-cs, sx, acc));
