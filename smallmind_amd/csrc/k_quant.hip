@@ -17,7 +17,7 @@ constexpr int kThreads = 256;
 __device__ __forceinline__ float rd_half_exact(const uint8_t *p) { return h2f_exact(ld_u16(p)); }
 
 // The codecs are bound by memory: 4 bytes per element on one side, and a block's bytes on the other.
-// A thread takes 4 elements, so that a wave reads or writes 1 KB of floats at once and the bytes of its
+// A thread takes 4 elements (8 of an 8-bit encoder), so that a wave reads or writes 1 KB of floats at once and the bytes of its
 // blocks (one K-quant block, eight of the 32-element ones) together; headers are read by all lanes of a
 // block from the same line, and an encoder's maxima are reduced over the lanes of its block.  Of 11.5 M
 // elements of Q4_K (53 MB each way, 10.6 us at the 5.0 TB/s of a large copy), one thread per block or
@@ -42,6 +42,9 @@ struct Type {
     static constexpr int bytes = T == SMX_TYPE_F32 ? 16 : T == SMX_TYPE_F16 ? 8 : T == SMX_TYPE_Q8_0 ? 34
                                : T == SMX_TYPE_Q4_0 ? 18 : T == SMX_TYPE_Q4_K ? 144 : T == SMX_TYPE_Q5_K ? 176
                                : T == SMX_TYPE_Q6_K ? 210 : T == SMX_TYPE_SMQ_Q8 ? 36 : 20;
+    // elements per thread of the encoder (8-bit codes: 8, half as many stores, which lie at odd addresses; 51 M
+    // elements of Q8_0, one thread per block / 4 / 8 elements per thread: 38 / 44 / 35 us)
+    static constexpr int enc = T == SMX_TYPE_Q8_0 || T == SMX_TYPE_SMQ_Q8 ? 8 : 4;
 };
 
 // ---- GGUF dequantization --------------------------------------------------------------------
@@ -124,13 +127,13 @@ __device__ __forceinline__ float group_max(float m)
     return m;
 }
 
-// Largest magnitude of the group's elements, NaN left out
-template <int G>
+// Largest magnitude of the group's elements (E per lane), NaN left out
+template <int G, int E = 4>
 __device__ __forceinline__ float group_maxabs(const float *x)
 {
     float m = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) { const float a = fabsf(x[i]); if (a > m) m = a; }
+    for (int i = 0; i < E; i++) { const float a = fabsf(x[i]); if (a > m) m = a; }
     return group_max<G>(m);
 }
 
@@ -148,25 +151,30 @@ template <int T>
 __device__ __forceinline__ void encode32(const float *x, int v, uint8_t *b)
 {
     constexpr bool q8 = T == SMX_TYPE_Q8_0 || T == SMX_TYPE_SMQ_Q8, smq = T == SMX_TYPE_SMQ_Q8 || T == SMX_TYPE_SMQ_Q4;
-    constexpr int head = smq ? 4 : 2;
-    const float maxAbs = group_maxabs<8>(x);
+    constexpr int head = smq ? 4 : 2, E = Type<T>::enc;
+    const float maxAbs = group_maxabs<32 / E, E>(x);
     const float scale = maxAbs > 0.0f ? maxAbs / (q8 ? 127.0f : 7.0f) : 1.0f;
     const float inv = 1.0f / scale;
     if (v == 0) {
         if (smq) st_any<uint32_t>(b, __float_as_uint(scale));
         else st_any<uint16_t>(b, (uint16_t)f2h_rne(scale));
     }
-    int c[4];
+    int c[E];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < E; i++) {
         const float t = x[i] * inv;
         c[i] = (int)rintf(clampf(t, q8 ? -127.0f : -8.0f, q8 ? 127.0f : 7.0f));
     }
-    if (q8)
-        st_any<uint32_t>(b + head + v, (uint32_t)(c[0] & 255) | (uint32_t)(c[1] & 255) << 8 |
-                                           (uint32_t)(c[2] & 255) << 16 | (uint32_t)(c[3] & 255) << 24);
-    else
+    if constexpr (q8) {
+        struct { uint32_t w[E / 4]; } o;
+#pragma unroll
+        for (int i = 0; i < E; i += 4)
+            o.w[i / 4] = (uint32_t)(c[i] & 255) | (uint32_t)(c[i + 1] & 255) << 8 | (uint32_t)(c[i + 2] & 255) << 16 |
+                         (uint32_t)(c[i + 3] & 255) << 24;
+        __builtin_memcpy(b + head + v, &o, E);
+    } else {
         st_any<uint16_t>(b + head + v / 2, (uint16_t)((c[0] & 15) | (c[1] & 15) << 4 | (c[2] & 15) << 8 | (c[3] & 15) << 12));
+    }
 }
 
 // d, dmin and the packed scales of a K-quant block, by the lane of its first element
@@ -263,17 +271,21 @@ __device__ __forceinline__ void encode_q6_k(const float *x, int v, uint8_t *b)
 template <int T>
 __global__ void k_quantize(const float *__restrict__ x, int64_t n, uint8_t *__restrict__ out)
 {
-    const int64_t e0 = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    constexpr int E = Type<T>::enc;
+    const int64_t e0 = E * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
     if (e0 >= n) return;   // whole groups of lanes: blocks are multiples of 32 elements
     uint8_t *b = out + e0 / Type<T>::elems * Type<T>::bytes;
     const int v = (int)(e0 % Type<T>::elems);
-    float f[4];
-    if (e0 + 4 <= n && ((uintptr_t)x & 15) == 0) {
-        const float4 q = *(const float4 *)(x + e0);
-        f[0] = q.x, f[1] = q.y, f[2] = q.z, f[3] = q.w;
+    float f[E];
+    if (e0 + E <= n && ((uintptr_t)x & 15) == 0) {
+#pragma unroll
+        for (int i = 0; i < E; i += 4) {
+            const float4 q = *(const float4 *)(x + e0 + i);
+            f[i] = q.x, f[i + 1] = q.y, f[i + 2] = q.z, f[i + 3] = q.w;
+        }
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; i++) f[i] = e0 + i < n ? x[e0 + i] : 0.0f;
+        for (int i = 0; i < E; i++) f[i] = e0 + i < n ? x[e0 + i] : 0.0f;
     }
     if constexpr (T == SMX_TYPE_Q4_K) {
         encode_q4_k(f, v, b);
@@ -448,7 +460,7 @@ hipError_t launch_quantize_gguf(int type, const float *x, int64_t n, void *block
         if constexpr (T != SMX_TYPE_F32)
             for (int64_t e = 0; e < n; e += kLaunchElems) {
                 const int64_t m = n - e < kLaunchElems ? n - e : kLaunchElems;
-                hipLaunchKernelGGL((k_quantize<T>), dim3(grid_for((m + 3) / 4)), dim3(kThreads), 0, s, x + e, m,
+                hipLaunchKernelGGL((k_quantize<T>), dim3(grid_for((m + Type<T>::enc - 1) / Type<T>::enc)), dim3(kThreads), 0, s, x + e, m,
                                    (uint8_t *)blocks + e / Type<T>::elems * Type<T>::bytes);
             }
     });
