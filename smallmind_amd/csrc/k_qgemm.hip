@@ -1356,6 +1356,8 @@ bool qgemm_tiled(const WView &w, int M)
     if (w.fmt == FMT_Q6_K || (narrow && (w.fmt != FMT_SQ8 || K >= 2048))) return S > 256;   // (SQ8: 4 waves)
     if (K >= 4096) return S >= 352;
     const bool offset = w.fmt == FMT_Q4_0 || w.fmt == FMT_SQ4;
+    // (fp32 scales cost the tile kernel's first part of a step: 11264 x 2048 SMQ Q4 65 tokens 35 / 37, 161 53 / 59)
+    if (w.fmt == FMT_SQ4 && tall && K >= 2048 && ((G > 256 && G <= 352) || (G > 512 && G <= 530))) return false;
     return S > (K >= 2048 ? (tall && offset ? 512 : 352) : offset ? 704 : 512);
 }
 
